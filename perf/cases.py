@@ -471,13 +471,13 @@ def tolerance(case):
     if fam == "matvec":
         return {"rel": 1e-13, "max": 1e-12} if case["dtype"] == "f64" else {"rel": 2e-6, "max": 1e-4}
     if _null_free(case):
-        return {"rel": 3e-2, "max": 0.5}
-    if fam in ("solve", "batch", "solve3d"):     # solves to a relative residual of 1e-8
-        return {"rel": 4e-6, "max": 4e-5}
-    if fam == "projection":
-        return {"rel": 4e-6, "max": 4e-5}
+        return {"rel": 3e-2, "max": 0.5} if case["mode"] == "nn" else {"rel": 2e-3, "max": 2e-2}
+    # solves to a relative residual of 1e-8; another summation order moves x by
+    # up to 2e-7, and a step's fields (the bubble's small momenta) by up to 4e-5
+    if fam in ("solve", "batch", "solve3d", "projection"):
+        return {"rel": 2e-6, "max": 1e-5}
     if fam in ("step", "ensemble"):
-        return {"rel": 1e-6, "max": 1e-4}
+        return {"rel": 1.7e-4, "max": 4e-4}
     if fam == "letkf":
         return {"rel": 1e-11, "max": 1e-9}
     return {"rel": 1e-2, "max": 0.2}             # BF16 network
