@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <string>
@@ -19,6 +20,8 @@ struct pb_ctx {
   double* scratch = nullptr;
   size_t scratch_bytes = 0;
   int scratch_err = 0;   // hipError_t of the address lookup
+  // Krylov runs to do by launches, after a resident run's wait ran out
+  std::atomic<int> resident_skip{0};
 };
 
 // Record a formatted error on the context and return code.
@@ -53,15 +56,31 @@ __device__ __forceinline__ double dpp_f64(double v) {
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
+// v plus the value of the lane at xor distance 32 (SWAP 32) or 16: the
+// exchange is one VALU swap per 32-bit half (v_permlane32_swap,
+// v_permlane16_swap) instead of a trip through LDS.  Swapping a register with
+// itself leaves the two halves' values in the two results, for every lane.
+template <int SWAP>
+__device__ __forceinline__ double add_swapped(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+  const auto l = SWAP == 32 ? __builtin_amdgcn_permlane32_swap(lo, lo, false, false)
+                            : __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  const auto h = SWAP == 32 ? __builtin_amdgcn_permlane32_swap(hi, hi, false, false)
+                            : __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  return __longlong_as_double(((long long)h[0] << 32) | (long long)l[0]) +
+         __longlong_as_double(((long long)h[1] << 32) | (long long)l[1]);
+}
+
 // Sum over the 64 lanes of a wave (every lane active), valid in lane 0.  The
 // order is the xor butterfly's: lane 0 adds the partial sum at xor distance
-// 32, 16, 8, 4, 2, 1 in turn.  The two cross-row steps go through
-// ds_bpermute; the four row-local ones are DPP moves.  After the distance-8
-// step lanes i and i^8 hold equal sums, so the row rotation by 4 delivers
-// the distance-4 partner's value whichever way it rotates.
+// 32, 16, 8, 4, 2, 1 in turn; the steps are register swaps and DPP moves.
+// After the distance-8 step lanes i and i^8 hold equal sums, so the row
+// rotation by 4 delivers the distance-4 partner's value whichever way it
+// rotates.
 __device__ __forceinline__ double wave_sum(double v) {
-  v += __shfl_xor(v, 32, kWave);
-  v += __shfl_xor(v, 16, kWave);
+  v = add_swapped<32>(v);
+  v = add_swapped<16>(v);
   v += dpp_f64<0x128>(v);   // row_ror 8: lane i ^ 8
   v += dpp_f64<0x124>(v);   // row_ror 4: lane i ^ 4 or i ^ 12 (equal sums)
   v += dpp_f64<0x4E>(v);    // quad_perm [2,3,0,1]: lane i ^ 2
@@ -69,20 +88,14 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// wave_sum of NV values at once, step by step over all values, so the
-// cross-row exchanges of the NV values are in flight together instead of
-// one round trip after another.  Same order of additions as wave_sum.
+// wave_sum of NV values at once, step by step over all values, so their
+// chains interleave.  Same order of additions as wave_sum.
 template <int NV>
 __device__ __forceinline__ void wave_sum_n(double (&v)[NV]) {
-  double t[NV];
 #pragma unroll
-  for (int k = 0; k < NV; ++k) t[k] = __shfl_xor(v[k], 32, kWave);
+  for (int k = 0; k < NV; ++k) v[k] = add_swapped<32>(v[k]);
 #pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] += t[k];
-#pragma unroll
-  for (int k = 0; k < NV; ++k) t[k] = __shfl_xor(v[k], 16, kWave);
-#pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] += t[k];
+  for (int k = 0; k < NV; ++k) v[k] = add_swapped<16>(v[k]);
 #pragma unroll
   for (int k = 0; k < NV; ++k) v[k] += dpp_f64<0x128>(v[k]);
 #pragma unroll

@@ -26,27 +26,12 @@
 #include <cstdlib>
 #include <type_traits>
 
-#include "pb_op2d.hpp"
+#include "pb_resident2d.hpp"
 
 using namespace pb2d;
 
 namespace {
 
-__device__ __forceinline__ double eps2() { return 4.930380657631324e-32; }   // DBL_EPSILON^2
-
-__device__ __forceinline__ int block_id() { return blockIdx.x + blockIdx.y * gridDim.x; }
-__device__ __forceinline__ int nblocks() { return gridDim.x * gridDim.y; }
-
-// XCD-aware tile order.  Hardware block h is dispatched to XCD h mod 8 (8
-// XCDs, each with its own L2).  Giving XCD x the contiguous tile range
-// [start(x), start(x) + count(x)) keeps vertically adjacent tiles, which share
-// halo rows, in one L2.  Bijective on [0, n); partial records stay indexed by
-// the tile number, so sums and iterates do not depend on the mapping.
-__device__ __forceinline__ int xcd_tile(int h, int n) {
-  constexpr int NX = 8;
-  const int x = h % NX, k = h / NX, base = n / NX, rem = n % NX;
-  return x < rem ? x * (base + 1) + k : rem * (base + 1) + (x - rem) * base + k;
-}
 __device__ __forceinline__ int thread_id() { return threadIdx.x + threadIdx.y * blockDim.x; }
 
 // ---------------------------------------------------------------------------
@@ -113,102 +98,6 @@ template <typename T, bool CROSS, bool CENTER, int RY>
 __global__ __launch_bounds__(NTHR) void k_init2(OpDev<T> op, InitIn<T> in, InitOut<T> out, double* P) {
   const int tile = xcd_tile(block_id(), nblocks());
   init_body<2, T, CROSS, CENTER, RY>(op, in, out, P, tile % gridDim.x, tile / gridDim.x, tile, nblocks());
-}
-
-// ---------------------------------------------------------------------------
-// scalar steps shared by every block
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ KState scalars_after_init(KState st, double rr, double bb) {
-  st.bnrm2 = sqrt(bb);
-  st.rnorm0 = sqrt(rr);
-  st.resid = st.rnorm0;
-  st.iter = 0;
-  st.half = 0;
-  st.alpha = 0.0;
-  st.omega = 0.0;
-  st.beta = 0.0;
-  st.x_upd = 0;
-  st.rho = rr;
-  st.atol = st.tol * st.bnrm2;
-  if (st.legacy ? (st.rnorm0 <= st.tol) : (st.rnorm0 <= st.atol)) {
-    st.status = ST_CONV;
-  } else if (fabs(rr) < eps2()) {
-    st.status = ST_BRK_RHO;
-  } else {
-    st.status = ST_RUN;
-  }
-  return st;
-}
-
-__device__ __forceinline__ KState scalars_after_b(KState st, const double (&tot)[5]) {
-  const double ss = tot[0], ts = tot[1], tt = tot[2], rts = tot[3], rtt = tot[4];
-  const double snrm = sqrt(ss);
-  st.x_upd = 1;
-  if (snrm <= st.atol) {
-    st.status = ST_P_HALF;
-    st.resid = snrm;
-    return st;
-  }
-  const double om = ts / tt;
-  if (!isfinite(om) || !isfinite(snrm)) {
-    st.status = ST_BRK_OMEGA;
-    return st;
-  }
-  st.omega = om;
-  const double rr = ss - 2.0 * om * ts + om * om * tt;
-  const double rho_new = rts - om * rtt;
-  st.iter += 1;
-  st.resid = sqrt(fmax(rr, 0.0));
-  if (st.resid <= st.atol) {
-    st.status = ST_P_CONV;
-  } else if (fabs(om) < eps2()) {
-    st.status = ST_P_BRK_OMEGA;
-  } else if (st.iter >= st.maxiter) {
-    st.status = ST_P_MAXIT;
-  } else {
-    const double beta = (rho_new / st.rho) * (st.alpha / om);
-    st.rho = rho_new;
-    if (fabs(rho_new) < eps2() || !isfinite(beta)) {
-      st.status = ST_P_BRK_RHO;
-    } else {
-      st.beta = beta;
-      st.status = ST_RUN;
-    }
-  }
-  return st;
-}
-
-__device__ __forceinline__ KState scalars_after_l3(KState st, double rtr, double rr) {
-  const double rnrm = sqrt(rr);
-  st.iter += 1;
-  st.resid = rnrm;
-  if (!isfinite(rnrm) || !isfinite(rtr)) {
-    st.status = ST_BRK_RHO;
-  } else if (rnrm <= st.atol) {
-    st.status = ST_CONV;
-  } else if (fabs(st.omega) < eps2()) {
-    st.status = ST_BRK_OMEGA;
-  } else if (st.iter >= st.maxiter) {
-    st.status = ST_MAXIT;
-  } else if (fabs(rtr) < eps2()) {
-    st.status = ST_BRK_RHO;
-  } else {
-    st.beta = (rtr / st.rho) * (st.alpha / st.omega);
-    st.rho = rtr;
-    st.status = ST_RUN;
-  }
-  return st;
-}
-
-__device__ __forceinline__ int finalize(int pending) {
-  switch (pending) {
-    case ST_P_CONV: return ST_CONV;
-    case ST_P_HALF: return ST_CONV;
-    case ST_P_MAXIT: return ST_MAXIT;
-    case ST_P_BRK_RHO: return ST_BRK_RHO;
-    case ST_P_BRK_OMEGA: return ST_BRK_OMEGA;
-    default: return pending;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1351,16 +1240,7 @@ int krylov_run(pb_op2d* op, Work<T>& w, const T* b, const double* x0, double tol
     return pb_fail(ctx, PB_ERR_ARG, "bicgstab: the one-launch iteration is FP64 only");
   const bool exact = variant == VAR_EXACT, fused = variant == VAR_FUSED;
   KState* hs = host ? host : op->hstate;
-  KState init{};
-  init.tol = tol;
-  init.maxiter = maxiter;
-  init.legacy = legacy;
-  init.status = ST_RUN;
-  init.phase = PH_INIT;
-  // the first launch of an iteration reads S0 (fast) or S2 (exact); the
-  // record travels as a kernel argument
-  hipLaunchKernelGGL(k_put_state, dim3(1), dim3(1), 0, s, w.S + (exact ? 2 : 0), init);
-  {
+  auto launch_init = [&] {
     // the one-launch iteration's adjoint launch sums the init records over
     // its own tiling
     const int iry = fused ? fused_ry(op) : op->ry;
@@ -1371,7 +1251,27 @@ int krylov_run(pb_op2d* op, Work<T>& w, const T* b, const double* x0, double tol
     const bool _c = op->cross, _h = op->center;
     if (exact) PB_RY_SWITCH(iry, PB_DISPATCH_AT, k_init2, T, grd, s, d, in, o, w.PC);
     else PB_RY_SWITCH(iry, PB_DISPATCH_AT, k_init5, T, grd, s, d, in, o, w.PB);
+  };
+  if (!host && !fused) {
+    // a grid whose tiles are all resident iterates in one launch; the init
+    // launch forms b - A x0 when a guess is given
+    if (x0) launch_init();
+    const ResJob<T> job{op, b, x0 ? w.r[0] : b, x0 ? w.x : nullptr, w.x, tol, maxiter, legacy};
+    Resident* R = resident_of(op);
+    if (!R) return PB_ERR_HIP;
+    const int rc = resident_run<T>(ctx, R->records, &job, 1, exact, s, out);
+    if (rc != 0) return rc < 0 ? rc : PB_OK;
   }
+  KState init{};
+  init.tol = tol;
+  init.maxiter = maxiter;
+  init.legacy = legacy;
+  init.status = ST_RUN;
+  init.phase = PH_INIT;
+  // the first launch of an iteration reads S0 (fast) or S2 (exact); the
+  // record travels as a kernel argument
+  hipLaunchKernelGGL(k_put_state, dim3(1), dim3(1), 0, s, w.S + (exact ? 2 : 0), init);
+  launch_init();
   if (exact) {
     launch_l1<T>(op, w, 1, s);
   } else if (fused) {
@@ -1934,6 +1834,7 @@ struct pb_batch {
   std::map<long, hipGraphExec_t> graphs;   // key: precision, chunk
   std::vector<int> ry_captured;            // member launch signatures the graphs were captured with
   KState* hst = nullptr;                   // pinned, one per member
+  pb2d::ResRecords records;                // of the resident runs
   // a user-facing batch is split into groups (each a batch of its own) whose
   // working sets fit the Infinity Cache together; groups are solved in turn
   std::vector<pb_batch*> groups;
@@ -2213,6 +2114,27 @@ template <typename T>
 int krylov_batch(pb_batch* bt, const std::vector<char>& active, const std::vector<const T*>& b,
                  const std::vector<double>& tol, int maxiter, int legacy, int check_every, hipStream_t s,
                  std::vector<KState>& out) {
+  {   // every active member's run in resident launches, where they fit
+    std::vector<ResJob<T>> jobs;
+    std::vector<size_t> who;
+    for (size_t m = 0; m < bt->ops.size(); ++m) {
+      if (!active[m]) continue;
+      pb_op2d* op = bt->ops[m];
+      jobs.push_back(ResJob<T>{op, b[m], b[m], nullptr, work_of<T>(op).x, tol[m], maxiter, legacy});
+      who.push_back(m);
+    }
+    if (jobs.empty()) return PB_OK;
+    std::vector<KState> st(jobs.size());
+    const int rc = resident_run<T>(bt->ctx, bt->records, jobs.data(), (int)jobs.size(), false, s, st.data());
+    if (rc < 0) return rc;
+    if (rc == 1) {
+      KState parked{};
+      parked.status = ST_CONV;
+      out.assign(bt->ops.size(), parked);
+      for (size_t k = 0; k < who.size(); ++k) out[who[k]] = st[k];
+      return PB_OK;
+    }
+  }
   // one launch over every member's tiles when they share the launch signature
   if (flat_signature(bt) >= 0) return krylov_batch_flat<T>(bt, active, b, tol, maxiter, legacy, check_every, s, out);
   const size_t M = bt->ops.size();
@@ -2362,6 +2284,7 @@ void batch_group_free(pb_batch* bt) {
   for (hipEvent_t ev : bt->joins) (void)hipEventDestroy(ev);
   if (bt->fork) (void)hipEventDestroy(bt->fork);
   if (bt->hst) (void)hipHostFree(bt->hst);
+  bt->records.release();
   delete bt;
 }
 }  // namespace

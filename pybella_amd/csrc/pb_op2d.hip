@@ -9,6 +9,7 @@
 //   k_matvec      lap2D_gather_new              laplacian.py:546-746
 // The flux form of the operator and the tiling are described in pb_op2d.hpp.
 #include "pb_op2d.hpp"
+#include "pb_resident2d.hpp"
 
 using namespace pb2d;
 
@@ -208,6 +209,7 @@ extern "C" int pb_op2d_destroy(pb_op2d* op) {
     if (op->ctx->own_stream) (void)hipStreamSynchronize(op->ctx->own_stream);
   }
   pb_fgmres_release(op);
+  pb2d::resident_free(op);
   for (auto& kv : op->w64.graphs) (void)hipGraphExecDestroy(kv.second);
   for (auto& kv : op->w32.graphs) (void)hipGraphExecDestroy(kv.second);
   for (void* p : op->allocs) (void)hipFree(p);

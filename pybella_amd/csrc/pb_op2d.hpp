@@ -342,6 +342,8 @@ struct Work {
   std::map<int, hipGraphExec_t> graphs;   // (variant, chunk) key -> instantiated graph
 };
 
+struct Resident;   // buffers of the runs that stay on the chip (pb_resident2d.hpp)
+
 }  // namespace pb2d
 
 namespace pbmg {
@@ -388,6 +390,7 @@ struct pb_op2d {
   pbmg::Hier* mg = nullptr;
   FgWork* fg = nullptr;
   pb_nn* nn = nullptr;
+  pb2d::Resident* res = nullptr;
 };
 
 namespace pb2d {
