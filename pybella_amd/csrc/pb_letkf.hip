@@ -9,197 +9,363 @@
 //   w   localisation weight / observation variance per observation (the
 //       weight is zero outside a wall);
 //   Pa  = (k-1)/rho I + Y^T diag(w) Y      (k x k, in the ensemble space)
-//   Pa  = V diag(lambda) V^T               (cyclic Jacobi, in LDS)
-//   Wa  = sqrt(k-1) V diag(lambda^-1/2) V^T + 1 wa^T,
-//   wa  = Pa^-1 Y^T diag(w) (y_obs - y_mean)
+//   Wa  = sqrt(k-1) Pa^-1/2 + 1 wa^T,   wa = Pa^-1 Y^T diag(w) (y_obs - y_mean)
 //   x_a^(i) = x_mean + sum_j Wa[i][j] (x^(j) - x_mean)  at the grid point.
 //
-// One 64-lane wave per grid point.  The window is streamed in chunks of 64
-// observation slots (one per lane) through LDS; masked slots carry weight 0.
+// Every contraction is on the FP64 matrix unit (v_mfma_f64_16x16x4: lane l
+// supplies A[l%16][l/16] and B[l/16][l%16] and holds D[l/16 + 4r][l%16], r =
+// 0..3).  A block analyses 8 x 4 points (2 x 4 above 16 members), a wave one
+// row of them, and stages the observation space of their windows attribute by
+// attribute in LDS, [position][member], the members' mean taken out once per
+// position instead of once per point and position.  Pa of a point is then one
+// matrix product per four observations, both operands from one LDS word per
+// lane; its inverse square root follows from scaled coupled Newton-Schulz
+// iterations (Higham, Functions of Matrices, 2008, sec. 6.7 and 8.3):
+//   X = Z Y, T = sqrt(s) (3 I - s X) / 2, Y <- Y T, Z <- T Z,
+// from Y = Pa / c, Z = I with c the largest column sum, Z -> sqrt(c) Pa^-1/2.
+// All spectra lie in [l, 1], l = (k-1) / (rho c) at first, so the scaling s =
+// 3 / (1 + sqrt(l) + l), which maps both ends of the interval to the same
+// value, is known in advance; l grows ~6x per iteration while it is small, and
+// 7 to 10 iterations reach rounding.  The registers of D are the right operand
+// of the next product as they stand and the left operand of its transpose, so
+// every iterate is kept with its transpose, at twice the products and without
+// a word through LDS.  (Taking a symmetric iterate's own registers for its
+// transpose's loses the iteration's stability: the error grows to 1e-3 at a
+// condition number of 1e4 instead of 2e-12.)
+//
+// Bound by the matrix unit: per point 2 * 16 * 16 flops per observation and
+// ~50 products of 16 x 16 matrices, 9 Gflop at 160 x 80 points, 4
+// attributes, 11 x 11 windows, 16 members (0.13 ms at the 73 Tflop/s of a large
+// product).  Both grid types of 161 x 81
+// (cells with 4 attributes, nodes with 1) take 0.50 ms; one wave per point with a
+// cyclic Jacobi eigendecomposition in LDS, 120 dependent rotations a sweep, took
+// 7.6 ms.
 // Layout: state and analysis (members, attrs, ny, nx), obs and mask
 // (attrs, ny, nx), x fastest; loc (obs_x, obs_y) row-major.
 #include "pb_common.hpp"
 
 namespace {
 
-constexpr int kLw = 64;   // lanes per grid point
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+constexpr int kWaves = 4;   // waves of a block, one per row of points
 
 struct LetkfArgs {
   int k, attrs, nx, ny, ox, oy, px, py, wall_x, wall_y;
   double rho;
 };
 
-template <int KM>
-__global__ __launch_bounds__(kLw) void k_letkf(LetkfArgs a, const double* __restrict__ state,
-                                               const double* __restrict__ obs, const double* __restrict__ mask,
-                                               const double* __restrict__ covar, const double* __restrict__ loc,
-                                               double* __restrict__ out) {
-  __shared__ double Ys[kLw][KM + 1];   // a chunk of observation anomalies [slot][member]
-  __shared__ double ws[kLw], inn[kLw];
-  __shared__ double A[KM][KM + 1], V[KM][KM + 1];
-  __shared__ double dv[KM], zv[KM], wav[KM], ls[KM];
-  const int lane = threadIdx.x;
-  const int pt = blockIdx.x;
-  const int ix = pt % a.nx, iy = pt / a.nx;
+// KT 16-member tiles; P points of a wave; CAP window positions staged at once
+template <int KT>
+struct LetkfShape {
+  static constexpr int P = KT == 1 ? 8 : 2;
+  static constexpr int CAP = KT == 1 ? 288 : 192;
+  static constexpr int S = 16 * KT + 1;   // members of a position, padded to an odd stride
+};
+
+__device__ __forceinline__ double over_groups(double v) {   // sum over the four 16-lane groups
+  v += __shfl_xor(v, 16);
+  return v + __shfl_xor(v, 32);
+}
+
+// A matrix of KT x KT register tiles, block (I, J) as the matrix unit's D
+template <int KT>
+struct Mat {
+  d4 b[KT][KT];
+};
+
+// A B from the registers of A^T and B.  As (A B)^T = B^T A^T, the transpose of
+// the product is mul(B, At), bit for bit.
+template <int KT>
+__device__ __forceinline__ Mat<KT> mul(const Mat<KT>& At, const Mat<KT>& B) {
+  Mat<KT> C;
+#pragma unroll
+  for (int I = 0; I < KT; ++I)
+#pragma unroll
+    for (int J = 0; J < KT; ++J) {
+      d4 c = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int K = 0; K < KT; ++K)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f64_16x16x4f64(At.b[K][I][r], B.b[K][J][r], c, 0, 0, 0);
+      C.b[I][J] = c;
+    }
+  return C;
+}
+
+// A v, v and the result as member J 16 + lane % 16 in every group
+template <int KT>
+__device__ __forceinline__ void mul_vec(const Mat<KT>& A, const double (&v)[KT], double (&w)[KT]) {   // A symmetric
+  const int row = threadIdx.x / 16;
+#pragma unroll
+  for (int J = 0; J < KT; ++J) w[J] = 0.0;
+#pragma unroll
+  for (int I = 0; I < KT; ++I)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const double x = __shfl(v[I], row + 4 * r);
+#pragma unroll
+      for (int J = 0; J < KT; ++J) w[J] += A.b[I][J][r] * x;
+    }
+#pragma unroll
+  for (int J = 0; J < KT; ++J) w[J] = over_groups(w[J]);
+}
+
+template <int KT>
+__global__ __launch_bounds__(64 * kWaves) void k_letkf(LetkfArgs a, int chunk_w, int chunk_h,
+                                                       const double* __restrict__ state,
+                                                       const double* __restrict__ obs, const double* __restrict__ mask,
+                                                       const double* __restrict__ covar, const double* __restrict__ loc,
+                                                       double* __restrict__ out) {
+  using H = LetkfShape<KT>;
+  constexpr int P = H::P, S = H::S;
+  __shared__ double Ys[H::CAP * S];          // observation anomalies [position][member]
+  __shared__ double wv[H::CAP], dv[H::CAP];  // 1 / deviation (0: not observed, outside a wall); innovation
+  const int lane = threadIdx.x, wave = threadIdx.y, tid = lane + 64 * wave;
+  const int m = lane % 16, grp = lane / 16;
+  const int tiles_x = (a.nx + P - 1) / P;
+  const int i0 = (blockIdx.x % tiles_x) * P, j0 = (blockIdx.x / tiles_x) * kWaves;
   const int k = a.k;
   const long plane = (long)a.nx * a.ny;
-  constexpr int EPL = (KM * KM + kLw - 1) / kLw;   // Pa entries per lane
-  double acc[EPL];
+  Mat<KT> acc[P];
+  double dacc[P][KT];
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) acc[e] = 0.0;
-  double dacc = 0.0;
-  const int nslot = a.attrs * a.ox * a.oy;
-  for (int base = 0; base < nslot; base += kLw) {
-    const int s = base + lane;
-    double w = 0.0, iv = 0.0;
-    if (s < nslot) {
-      const int at = s / (a.ox * a.oy), r = s % (a.ox * a.oy), wx = r / a.oy, wy = r % a.oy;
-      const int ux = ix + wx - a.px, uy = iy + wy - a.py;
-      const int gx = ((ux % a.nx) + a.nx) % a.nx, gy = ((uy % a.ny) + a.ny) % a.ny;
-      const long g = (long)gy * a.nx + gx;
-      if (mask[at * plane + g] == 0.0) {
-        double sum = 0.0;
-        for (int m = 0; m < k; ++m) sum += state[((long)m * a.attrs + at) * plane + g];
-        const double ym = sum / k;
-        for (int m = 0; m < k; ++m) Ys[lane][m] = state[((long)m * a.attrs + at) * plane + g] - ym;
-        const bool out_x = a.wall_x && (ux < 0 || ux >= a.nx), out_y = a.wall_y && (uy < 0 || uy >= a.ny);
-        const double L = (out_x || out_y) ? 0.0 : loc[wx * a.oy + wy];
-        w = L / (covar ? covar[at] : 1.0);
-        iv = obs[at * plane + g] - ym;
-      } else {
-        for (int m = 0; m < k; ++m) Ys[lane][m] = 0.0;
-      }
-    } else {
-      for (int m = 0; m < k; ++m) Ys[lane][m] = 0.0;
-    }
-    ws[lane] = w;
-    inn[lane] = iv;
-    __syncthreads();
-    const int cnt = min(kLw, nslot - base);
+  for (int p = 0; p < P; ++p)
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      const int idx = lane + e * kLw;
-      if (idx < k * k) {
-        // (lo, hi) order: the (p, q) and (q, p) sums are the same
-        // operations, so Pa is exactly symmetric
-        const int p = min(idx / k, idx % k), q = max(idx / k, idx % k);
-        double sacc = acc[e];
-        for (int j = 0; j < cnt; ++j) sacc += ws[j] * Ys[j][p] * Ys[j][q];
-        acc[e] = sacc;
-      }
-    }
-    if (lane < k)
-      for (int j = 0; j < cnt; ++j) dacc += ws[j] * Ys[j][lane] * inn[j];
-    __syncthreads();
-  }
-  // Pa and V = I
-  const double diag = (k - 1.0) / a.rho;
+    for (int I = 0; I < KT; ++I) {
+      dacc[p][I] = 0.0;
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) {
-    const int idx = lane + e * kLw;
-    if (idx < k * k) {
-      const int p = idx / k, q = idx % k;
-      A[p][q] = (p == q ? diag : 0.0) + acc[e];
-      V[p][q] = p == q ? 1.0 : 0.0;
+      for (int J = 0; J < KT; ++J) acc[p].b[I][J] = d4{0.0, 0.0, 0.0, 0.0};
     }
-  }
-  if (lane < k) dv[lane] = dacc;
-  __syncthreads();
-  // cyclic Jacobi sweeps (Golub & Van Loan, Alg. 8.5.2 with the symmetric
-  // Schur rotation) until the off-diagonal part is negligible: V collects
-  // the rotations, the diagonal of A becomes the eigenvalues
-  for (int sweep = 0; sweep < 40; ++sweep) {
-    double off = 0.0, dg = 0.0;
-    if (lane < k)
-      for (int q = 0; q < k; ++q) {
-        const double v = A[lane][q];
-        if (q == lane) dg += v * v; else off += v * v;
-      }
-    for (int o = 32; o > 0; o >>= 1) {
-      off += __shfl_xor(off, o);
-      dg += __shfl_xor(dg, o);
-    }
-    if (!(off > 1e-30 * dg)) break;
-    for (int p = 0; p < k - 1; ++p)
-      for (int q = p + 1; q < k; ++q) {
-        const double apq = A[p][q];
-        if (apq == 0.0) continue;
-        const double app = A[p][p], aqq = A[q][q];
-        const double tau = (aqq - app) / (2.0 * apq);
-        const double t = (tau >= 0.0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
-        const double c = 1.0 / sqrt(1.0 + t * t), sn = t * c;
-        double arp = 0.0, arq = 0.0, vrp = 0.0, vrq = 0.0;
-        if (lane < k) {
-          arp = A[lane][p];
-          arq = A[lane][q];
-          vrp = V[lane][p];
-          vrq = V[lane][q];
-        }
+
+  // Y^T W Y and Y^T W d over the windows, by attribute, by chunks of
+  // chunk_w window columns and of chunk_h rows of the block's window union
+  for (int at = 0; at < a.attrs; ++at) {
+    const double idev = 1.0 / sqrt(covar ? covar[at] : 1.0);
+    for (int c0 = 0; c0 < a.ox; c0 += chunk_w) {
+      const int cw = min(chunk_w, a.ox - c0), RW = P + cw - 1;
+      for (int r0 = 0; r0 < kWaves + a.oy - 1; r0 += chunk_h) {
+        const int rh = min(chunk_h, kWaves + a.oy - 1 - r0);
         __syncthreads();
-        if (lane < k) {
-          if (lane == p) {
-            A[p][p] = app - t * apq;
-            A[p][q] = 0.0;
-            A[q][p] = 0.0;
-          } else if (lane == q) {
-            A[q][q] = aqq + t * apq;
-          } else {
-            const double np_ = c * arp - sn * arq, nq_ = sn * arp + c * arq;
-            A[lane][p] = np_;
-            A[p][lane] = np_;
-            A[lane][q] = nq_;
-            A[q][lane] = nq_;
+        for (int s = tid; s < RW * rh; s += 64 * kWaves) {
+          const int ux = i0 + c0 + s % RW - a.px, uy = j0 + r0 + s / RW - a.py;
+          const int gx = ((ux % a.nx) + a.nx) % a.nx, gy = ((uy % a.ny) + a.ny) % a.ny;
+          const long g = at * plane + (long)gy * a.nx + gx;
+          double* y = Ys + s * S;
+          const bool seen = mask[g] == 0.0;
+          double sum = 0.0;
+          if (seen) {
+            const double* f = state + g;
+#pragma unroll 8
+            for (int q = 0; q < k; ++q) {
+              const double v = f[q * a.attrs * plane];
+              y[q] = v;
+              sum += v;
+            }
           }
-          V[lane][p] = c * vrp - sn * vrq;
-          V[lane][q] = sn * vrp + c * vrq;
+          const double ym = sum / k;
+          for (int q = 0; q < 16 * KT; ++q) y[q] = (seen && q < k) ? y[q] - ym : 0.0;
+          const bool outside = (a.wall_x && (ux < 0 || ux >= a.nx)) || (a.wall_y && (uy < 0 || uy >= a.ny));
+          wv[s] = (seen && !outside) ? idev : 0.0;
+          dv[s] = seen ? obs[g] - ym : 0.0;
         }
         __syncthreads();
-      }
-  }
-  // z_e = (V^T d)_e / lambda_e, wa = V z; ls = sqrt(1 / lambda)
-  if (lane < k) {
-    double z = 0.0;
-    for (int i = 0; i < k; ++i) z += V[i][lane] * dv[i];
-    zv[lane] = z * (1.0 / A[lane][lane]);
-    ls[lane] = sqrt(1.0 / A[lane][lane]);
-  }
-  __syncthreads();
-  if (lane < k) {
-    double w = 0.0;
-    for (int e = 0; e < k; ++e) w += V[lane][e] * zv[e];
-    wav[lane] = w;
-  }
-  __syncthreads();
-  // Wa = sqrt(k-1) V diag(sqrt(1/lambda)) V^T + wa, into the A storage
-  const double sk = sqrt(k - 1.0);
+        if (j0 + wave >= a.ny) continue;
+        // this row's window rows in the chunk, four observations at a time
+        const int w0 = max(0, r0 - wave), w1 = min(a.oy, r0 + rh - wave);
+        const int n = (w1 - w0) * cw;
+        int q = 0, c = grp;
+        while (c >= cw) {
+          c -= cw;
+          ++q;
+        }
+        auto weight = [&](int s) { return s < n ? loc[(c0 + c) * a.oy + w0 + q] : 0.0; };
+        double L = weight(grp);
+        for (int s = grp; s < n + grp; s += 4) {   // the same number of steps in every group
+          const bool ok = s < n;
+          const int pos = ok ? (wave + w0 + q - r0) * RW + c : 0;
+          // both operands carry the root of the weight, so Pa is exactly
+          // symmetric; a negative weight's sign goes with one of them
+          const double rl = sqrt(fabs(L));
+          const bool neg = L < 0.0;
+          c += 4;
+          while (c >= cw) {
+            c -= cw;
+            ++q;
+          }
+          L = weight(s + 4);   // in flight during this step's products
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) {
-    const int idx = lane + e * kLw;
-    if (idx < k * k) {
-      const int i = idx / k, j = idx % k;
-      double s = 0.0;
-      for (int f = 0; f < k; ++f) s += V[i][f] * ls[f] * V[j][f];
-      acc[e] = sk * s + wav[j];
+          for (int p = 0; p < P; ++p) {
+            const double w = rl * wv[pos + p], wd = ok ? w * dv[pos + p] : 0.0;
+            double y[KT], wy[KT];
+#pragma unroll
+            for (int I = 0; I < KT; ++I) {
+              y[I] = ok ? w * Ys[(pos + p) * S + 16 * I + m] : 0.0;
+              wy[I] = neg ? -y[I] : y[I];
+              dacc[p][I] += wy[I] * wd;
+            }
+#pragma unroll
+            for (int I = 0; I < KT; ++I)
+#pragma unroll
+              for (int J = 0; J < KT; ++J)
+                acc[p].b[I][J] = __builtin_amdgcn_mfma_f64_16x16x4f64(wy[I], y[J], acc[p].b[I][J], 0, 0, 0);
+          }
+        }
+      }
     }
   }
-  __syncthreads();
+  if (j0 + wave >= a.ny) return;
+
+  const double diag = (k - 1.0) / a.rho;
+#pragma unroll 1
+  for (int p = 0; p < P && i0 + p < a.nx; ++p) {
+    // Pa; the rows past the members are those of diag I
+    Mat<KT> Y, Yt, Z, Zt, T, Tt;   // with their transposes
+    double d[KT], big = 0.0;
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) {
-    const int idx = lane + e * kLw;
-    if (idx < k * k) A[idx / k][idx % k] = acc[e];
+    for (int q = 0; q < P; ++q) {   // acc[p] by a constant index
+      if (q == p) {
+        Y = acc[q];
+#pragma unroll
+        for (int I = 0; I < KT; ++I) d[I] = dacc[q][I];
+      }
+    }
+#pragma unroll
+    for (int J = 0; J < KT; ++J) {
+      double col = 0.0;
+#pragma unroll
+      for (int I = 0; I < KT; ++I)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (I == J && grp + 4 * r == m) Y.b[I][J][r] += diag;
+          col += fabs(Y.b[I][J][r]);
+        }
+      big = fmax(big, over_groups(col));
+      d[J] = over_groups(d[J]);
+    }
+    for (int o = 1; o < 16; o <<= 1) big = fmax(big, __shfl_xor(big, o));
+    const double ic = 1.0 / big;
+    double low = fmin(diag * ic, 1.0), dev0 = 1e300;
+#pragma unroll
+    for (int I = 0; I < KT; ++I)
+#pragma unroll
+      for (int J = 0; J < KT; ++J) Y.b[I][J] *= ic;
+    Yt = Y;
+    for (int it = 0; it < 80; ++it) {
+      T = it == 0 ? Y : mul<KT>(Zt, Y);
+      Tt = it == 0 ? Y : mul<KT>(Y, Zt);
+      // the planned iterations leave X within ~1e-9 of I; then on to where
+      // it no longer improves
+      const bool planned = 1.0 - low > 1e-9;
+      bool last = false;
+      if (!planned) {
+        double dev = 0.0;
+#pragma unroll
+        for (int I = 0; I < KT; ++I)
+#pragma unroll
+          for (int J = 0; J < KT; ++J)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              dev = fmax(dev, fabs(T.b[I][J][r] - ((I == J && grp + 4 * r == m) ? 1.0 : 0.0)));
+        for (int o = 1; o < 64; o <<= 1) dev = fmax(dev, __shfl_xor(dev, o));
+        last = dev < 1e-8 || (dev < 1e-2 && dev > 0.5 * dev0);
+        dev0 = dev;
+      }
+      const double sc = planned ? 3.0 / (1.0 + sqrt(low) + low) : 1.0, rs = sqrt(sc), hs = 0.5 * rs * sc;
+#pragma unroll
+      for (int I = 0; I < KT; ++I)
+#pragma unroll
+        for (int J = 0; J < KT; ++J)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const double e = (I == J && grp + 4 * r == m) ? 1.5 * rs : 0.0;
+            T.b[I][J][r] = e - hs * T.b[I][J][r];
+            Tt.b[I][J][r] = e - hs * Tt.b[I][J][r];
+          }
+      if (it == 0) {
+        Z = T;
+        Zt = Tt;
+      } else {
+        const Mat<KT> Zn = mul<KT>(Tt, Z);
+        Zt = mul<KT>(Z, Tt);
+        Z = Zn;
+      }
+      if (last) break;
+      const Mat<KT> Yn = mul<KT>(Yt, T);
+      Yt = mul<KT>(T, Yt);
+      Y = Yn;
+      low = fmin(0.25 * sc * low * (3.0 - sc * low) * (3.0 - sc * low), 1.0);
+    }
+    // Z = Pa^-1/2; wa = Pa^-1 d
+    const double rc = sqrt(ic);
+#pragma unroll
+    for (int I = 0; I < KT; ++I)
+#pragma unroll
+      for (int J = 0; J < KT; ++J) Z.b[I][J] *= rc;
+    double z[KT], wa[KT];
+    mul_vec<KT>(Z, d, z);
+    mul_vec<KT>(Z, z, wa);
+    // Wa as the left operand: row J 16 + m, column I 16 + grp + 4 r
+    const double sk = sqrt(k - 1.0);
+#pragma unroll
+    for (int I = 0; I < KT; ++I)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double w = __shfl(wa[I], grp + 4 * r);
+#pragma unroll
+        for (int J = 0; J < KT; ++J) Z.b[I][J][r] = sk * Z.b[I][J][r] + w;
+      }
+    // the analysis of up to 16 attributes at once: attribute a0 + m in column m
+    const long g = (long)(j0 + wave) * a.nx + i0 + p;
+    for (int a0 = 0; a0 < a.attrs; a0 += 16) {
+      const bool has = a0 + m < a.attrs;
+      const double* f = state + (has ? a0 + m : 0) * plane + g;
+      double x[KT][4], sum = 0.0;
+#pragma unroll
+      for (int I = 0; I < KT; ++I)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int mem = 16 * I + grp + 4 * r;
+          x[I][r] = (has && mem < k) ? f[(long)mem * a.attrs * plane] : 0.0;
+          sum += x[I][r];
+        }
+      const double xm = over_groups(sum) / k;
+#pragma unroll
+      for (int I = 0; I < KT; ++I)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[I][r] = (has && 16 * I + grp + 4 * r < k) ? x[I][r] - xm : 0.0;
+#pragma unroll
+      for (int J = 0; J < KT; ++J) {
+        d4 o = {xm, xm, xm, xm};
+#pragma unroll
+        for (int I = 0; I < KT; ++I)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o = __builtin_amdgcn_mfma_f64_16x16x4f64(Z.b[I][J][r], x[I][r], o, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int mem = 16 * J + grp + 4 * r;
+          if (has && mem < k) out[((long)mem * a.attrs + a0 + m) * plane + g] = o[r];
+        }
+      }
+    }
   }
-  __syncthreads();
-  // analysis at this grid point: member i, attribute at
-  const long g = (long)iy * a.nx + ix;
-  for (int idx = lane; idx < k * a.attrs; idx += kLw) {
-    const int i = idx / a.attrs, at = idx % a.attrs;
-    double sum = 0.0;
-    for (int m = 0; m < k; ++m) sum += state[((long)m * a.attrs + at) * plane + g];
-    const double xm = sum / k;
-    double s = 0.0;
-    for (int j = 0; j < k; ++j) s += A[i][j] * (state[((long)j * a.attrs + at) * plane + g] - xm);
-    out[((long)i * a.attrs + at) * plane + g] = s + xm;
+}
+
+template <int KT>
+void launch_letkf(const LetkfArgs& a, hipStream_t s, const double* state, const double* obs, const double* mask,
+                  const double* covar, const double* loc, double* out) {
+  using H = LetkfShape<KT>;
+  // the window union of the block, whole where it fits the staging area, else
+  // in chunks of whole rows, else of parts of rows
+  const int rows = kWaves + a.oy - 1;
+  int cw = a.ox, ch = H::CAP / (H::P + cw - 1);
+  if (ch < 1) {
+    ch = 1;
+    cw = H::CAP - H::P + 1;
   }
+  if (ch > rows) ch = rows;
+  const dim3 grid((unsigned)ceil_div(a.nx, H::P) * (unsigned)ceil_div(a.ny, kWaves));
+  hipLaunchKernelGGL(k_letkf<KT>, grid, dim3(64, kWaves), 0, s, a, cw, ch, state, obs, mask, covar, loc, out);
 }
 
 }  // namespace
@@ -220,13 +386,8 @@ extern "C" int pb_letkf_analyse(pb_ctx* ctx, const pb_letkf_cfg* cfg, const doub
   if ((long)cfg->nx * cfg->ny > (1L << 31) - 1) return pb_fail(ctx, PB_ERR_ARG, "pb_letkf_analyse: grid too large");
   LetkfArgs a{k, cfg->attrs, cfg->nx, cfg->ny, cfg->obs_x, cfg->obs_y, (cfg->obs_x - 1) / 2, (cfg->obs_y - 1) / 2,
               !cfg->periodic_x, !cfg->periodic_y, cfg->inflation};
-  const dim3 grid((unsigned)(cfg->nx * cfg->ny));
-  if (k <= 8)
-    hipLaunchKernelGGL(k_letkf<8>, grid, dim3(kLw), 0, ctx->stream, a, state, obs, mask, covar, loc, analysis);
-  else if (k <= 16)
-    hipLaunchKernelGGL(k_letkf<16>, grid, dim3(kLw), 0, ctx->stream, a, state, obs, mask, covar, loc, analysis);
-  else
-    hipLaunchKernelGGL(k_letkf<32>, grid, dim3(kLw), 0, ctx->stream, a, state, obs, mask, covar, loc, analysis);
+  if (k <= 16) launch_letkf<1>(a, ctx->stream, state, obs, mask, covar, loc, analysis);
+  else launch_letkf<2>(a, ctx->stream, state, obs, mask, covar, loc, analysis);
   PB_LAUNCH_CHECK(ctx);
   return PB_OK;
 }
