@@ -63,9 +63,12 @@ class LETKF:
         attribute or None).  Writes the analysis into the fields."""
         torch = _torch()
         k, na = len(fields), len(fields[0])
-        inner = [[f[2:-2, 2:-2] for f in mem] for mem in fields]
-        ny, nx = inner[0][0].shape
-        state = torch.stack([torch.stack(mem) for mem in inner]).contiguous()          # (k, attrs, ny, nx)
+        # every member field in one gather, and back in one scatter of padded
+        # fields: per field it took a fill and a strided copy, 2 k attrs launches
+        flat = [f for mem in fields for f in mem]
+        full = torch.stack(flat)
+        ny, nx = full.shape[1] - 4, full.shape[2] - 4
+        state = full[:, 2:-2, 2:-2].contiguous().view(k, na, ny, nx)
         dev = lambda a: torch.from_numpy(np.ascontiguousarray(np.asarray(a, dtype=np.float64))).cuda()
         obs_d = dev(np.stack([np.asarray(o).T for o in obs]))
         mask_d = dev(np.stack([np.asarray(m).T != 0 for m in mask]).astype(np.float64))
@@ -78,10 +81,9 @@ class LETKF:
         self.ctx.check(self.ctx.lib.pb_letkf_analyse(self.ctx.h, C.byref(cfg), _abi.ptr(state), _abi.ptr(obs_d),
                                                      _abi.ptr(mask_d), _abi.ptr(cov_d), _abi.ptr(loc_d),
                                                      _abi.ptr(out)), "pb_letkf_analyse")
-        for m, mem in enumerate(fields):
-            for a, f in enumerate(mem):
-                f.zero_()
-                f[2:-2, 2:-2].copy_(out[m, a])
+        full.zero_()
+        full[:, 2:-2, 2:-2] = out.view(k * na, ny, nx)
+        torch._foreach_copy_(flat, list(full.unbind(0)))
 
     def analyse(self, models, obs, mask, covar=None):
         """The analysis of the members' device states (time_update.DeviceModel
