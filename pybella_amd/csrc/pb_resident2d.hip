@@ -10,10 +10,12 @@
 // r~, x, diag_inv and the cell weights fit the register file (38 of its 128
 // MB at 1025x513), and what blocks exchange is one ring of edge values and a
 // few sums per stencil.  FP64 at 4-row tiles, us per iteration, launches ->
-// resident: two phases 14.0 -> 7.3 (161x81), 13.6 -> 10.2 (513x257), 24.7 ->
-// 15.4 (1025x513); the exact variant's three 18.7 -> 9.3, 18.5 -> 13.7, 28.5 ->
-// 20.0.  What is left is latency: per phase at 161x81 about 1.6 us for the
-// hand-over and 2 us for the chain combine, stencil, sums, scalars of one tile.
+// resident: two phases 14.0 -> 6.7 (161x81), 13.6 -> 9.8 (513x257), 24.7 ->
+// 15.0 (1025x513); the exact variant's three 18.7 -> 9.1, 18.5 -> 13.5, 28.5 ->
+// 19.6.  What is left is latency: per phase at 161x81 about 1.5 us for the
+// hand-over and 1.9 us for the chain combine, stencil, sums, scalars of one
+// tile.  (x updated in the chain instead of behind the hand-over: 7.3; eight
+// waves per tile instead of four: 6.8; waves that sleep between polls: 7.3.)
 //
 // Exchange.  Every word that crosses blocks carries its own tag: 8-byte
 // relaxed agent-scope atomics holding 32 bits of a value and the 32-bit
@@ -178,7 +180,10 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
   constexpr int TY = TYT * RY;
   constexpr int NW = NTHR / kWave;
   constexpr int W = Tagged<T>::W;
-  __shared__ T sp[(TY + 2) * (TX + 2)];   // the stencil's input with its ring
+  constexpr bool LATE = MINB == 2 && RY <= 4;   // registers to update x in while the words travel
+  // the stencil's input with its ring, and spare rows that take the stores of
+  // threads past the grid
+  __shared__ T sp[(TY + 2 + RY) * (TX + 2)];
   __shared__ T so[TY * TX];               // its output
   __shared__ double sred[5 * NW], ssum[5 * NW];
   // used once per phase by the thread they belong to, so kept off the registers
@@ -192,7 +197,7 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
     sdead = 0;
     sid = (int)(atomicAdd(ticket, 1u) - ticket0);
   }
-  for (int k = tid; k < (TY + 2) * (TX + 2); k += NTHR) sp[k] = T(0);
+  for (int k = tid; k < (TY + 2 + RY) * (TX + 2); k += NTHR) sp[k] = T(0);
   __syncthreads();
   const int blk = __builtin_amdgcn_readfirstlane(sid);
   int m = 0;
@@ -317,9 +322,10 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
   };
   auto stencil = [&](const T(&c)[RY], T h, T(&y)[RY]) {
     T* const row0 = sp + (ty * RY) * (TX + 2) + tx;   // left of the row above the own ones
+    T* const spare = sp + (TY + 2) * (TX + 2) + tx;
+    T* const own = tx < Wd ? row0 + (TX + 2) + 1 : spare;
 #pragma unroll
-    for (int q = 0; q < RY; ++q)
-      if (okm >> q & 1) row0[(q + 1) * (TX + 2) + 1] = c[q];
+    for (int q = 0; q < RY; ++q) (ty * RY + q < H ? own : spare)[q * (TX + 2)] = c[q];
     if (ring) sp[rpos] = h;
     __syncthreads();
     T left[RY + 2], mid[RY + 2], fx[RY + 1], fy[RY + 1], ex, ey;
@@ -351,7 +357,7 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
     for (int q = 0; q < RY; ++q) {
       T acc = ((fxr[q] + fxr[q + 1]) - (fx[q] + fx[q + 1])) + ((fy[q + 1] + fyr[q + 1]) - (fy[q] + fyr[q]));
       if (CENTER) acc = fma_(hv[q], c[q], acc);
-      y[q] = (okm >> q & 1) ? Ldv[q][tid] * acc : T(0);
+      y[q] = Ldv[q][tid] * acc;   // past the grid: unused
       so[(ty * RY + q) * TX + tx] = y[q];
     }
     __syncthreads();
@@ -359,9 +365,10 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
 
   // One phase's hand-over: the tile's edges out (from so) and the ring's
   // values in, if ``buf``; ``vals`` summed over every tile and given to
-  // ``scalars``, which advances the run's state sst.  REC: the phase's first
-  // record value.  False: a wait ran out.
-  auto exchange = [&](auto nv_, auto rec_, u64* buf, T* h, u32 tag, auto&& scalars) -> bool {
+  // ``scalars``, which advances the run's state sst.  ``meanwhile`` runs once
+  // the tile's words are out.  REC: the phase's first record value.  False: a
+  // wait ran out.
+  auto exchange = [&](auto nv_, auto rec_, u64* buf, T* h, u32 tag, auto&& meanwhile, auto&& scalars) -> bool {
     constexpr int NV = decltype(nv_)::value, REC = decltype(rec_)::value;
     constexpr int LAST = NW - 1;
     wave_sum_n<NV>(reinterpret_cast<double(&)[NV]>(vals));
@@ -387,6 +394,7 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
     } else if (buf && nb > 1) {
       publish(buf, tag);
     }
+    meanwhile();
     // The order of sum_partials: class w adds records 64 w + lane + 256 h,
     // then its lanes; the class sums are added in order of w.
     if (nb > kDirect) {
@@ -500,7 +508,7 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
       vals[1] = fma_(bd, bd, vals[1]);
     }
   }
-  if (!exchange(two, recC, nullptr, nullptr, ++tag, [](KState& st, const double(&tot)[2]) {
+  if (!exchange(two, recC, nullptr, nullptr, ++tag, [] {}, [](KState& st, const double(&tot)[2]) {
         st = scalars_after_init(st, tot[0], tot[1]);
         st.phase = PH_A;
       }))
@@ -520,20 +528,27 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
       break;
     }
     // A: p and v = A p
+    T xp[RY], xs[RY];   // the last iteration's p and s, for x
+    const double alpha_x = sst.alpha, omega_x = sst.omega;
+    const int xupd = !EXACT && sst.x_upd;
     {
-      const double alpha_d = sst.alpha, omega_d = sst.omega;
+      const double alpha_d = alpha_x, omega_d = omega_x;
       const T alpha = (T)alpha_d, omega = (T)omega_d, beta = (T)sst.beta;
       if (EXACT) {
 #pragma unroll
         for (int q = 0; q < RY; ++q) p[q] = fma_(beta, fma_(-omega, v[q], p[q]), r[q]);
         hp = fma_(beta, fma_(-omega, hvv, hp), hr);
       } else {
-        const int xupd = sst.x_upd;
 #pragma unroll
         for (int q = 0; q < RY; ++q) {
           const T s = fma_(-alpha, v[q], r[q]);
           const T rn = fma_(-omega, t[q], s);
-          if (xupd) Lx[q][tid] = fma_(omega_d, (double)s, fma_(alpha_d, (double)p[q], Lx[q][tid]));
+          if (LATE) {
+            xp[q] = p[q];
+            xs[q] = s;
+          } else if (xupd) {
+            Lx[q][tid] = fma_(omega_d, (double)s, fma_(alpha_d, (double)p[q], Lx[q][tid]));
+          }
           p[q] = fma_(beta, fma_(-omega, v[q], p[q]), rn);
           r[q] = rn;
         }
@@ -550,7 +565,14 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
       const int k = (ty + TYT * q) * TX + tx;
       if (oks >> q & 1) vals[0] = fma_((double)Lrt[k], (double)so[k], vals[0]);
     }
-    if (!exchange(one, recA, M.halo_v, &hvv, tag, [](KState& st, const double(&tot)[1]) {
+    auto update_x = [&] {
+      if (LATE && xupd) {
+#pragma unroll
+        for (int q = 0; q < RY; ++q)
+          Lx[q][tid] = fma_(omega_x, (double)xs[q], fma_(alpha_x, (double)xp[q], Lx[q][tid]));
+      }
+    };
+    if (!exchange(one, recA, M.halo_v, &hvv, tag, update_x, [](KState& st, const double(&tot)[1]) {
           const double alpha = st.rho / tot[0];
           st.phase = PH_B;
           if (tot[0] == 0.0 || !isfinite(alpha)) st.status = ST_BRK_OMEGA;
@@ -580,7 +602,7 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
         vals[4] = fma_(rd, yd, vals[4]);
       }
     }
-    if (!exchange(five, recB, M.halo_t, &ht, tag, [](KState& st, const double(&tot)[5]) {
+    if (!exchange(five, recB, M.halo_t, &ht, tag, [] {}, [](KState& st, const double(&tot)[5]) {
           if (!EXACT) {
             st = scalars_after_b(st, tot);
             st.phase = PH_A;
@@ -608,17 +630,15 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
     const bool half = sst.status == ST_P_HALF;
     const double omega_d = sst.omega;
     const T omega = (T)omega_d;
+    T sn[RY];
 #pragma unroll
     for (int q = 0; q < RY; ++q) {
-      const double xg = fma_(alpha_d, (double)p[q], Lx[q][tid]);
+      sn[q] = fma_(-alpha, v[q], r[q]);
       if (half) {
-        Lx[q][tid] = xg;
+        Lx[q][tid] = fma_(alpha_d, (double)p[q], Lx[q][tid]);
       } else {
-        const T s = fma_(-alpha, v[q], r[q]);
-        Lx[q][tid] = fma_(omega_d, (double)s, xg);
-        const T rn = fma_(-omega, t[q], s);
-        r[q] = rn;
-        so[(ty * RY + q) * TX + tx] = rn;
+        r[q] = fma_(-omega, t[q], sn[q]);
+        so[(ty * RY + q) * TX + tx] = r[q];
       }
     }
     if (half) break;
@@ -634,7 +654,12 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
         vals[1] = fma_(rn, rn, vals[1]);
       }
     }
-    if (!exchange(two, recC, nullptr, nullptr, ++tag, [](KState& st, const double(&tot)[2]) {
+    auto update_x_exact = [&] {
+#pragma unroll
+      for (int q = 0; q < RY; ++q)
+        Lx[q][tid] = fma_(omega_d, (double)sn[q], fma_(alpha_d, (double)p[q], Lx[q][tid]));
+    };
+    if (!exchange(two, recC, nullptr, nullptr, ++tag, update_x_exact, [](KState& st, const double(&tot)[2]) {
           st = scalars_after_l3(st, tot[0], tot[1]);
           st.phase = PH_A;
         }))
