@@ -38,7 +38,7 @@
 
 namespace {
 
-constexpr int X3 = 64, Y3 = 8, Z3 = 16;
+constexpr int X3 = 64, Y3 = 8, Z3 = 16;   // tile of a marching block; its z planes, unless a launch says otherwise
 constexpr int NT3 = X3 * Y3;   // threads of a marching block
 constexpr int kNV = 5;   // max partials per block
 
@@ -588,7 +588,7 @@ struct Iter1In {
 // x += alpha p + omega (r - alpha v), p_k = r_{k-1} + beta (p - omega v),
 // v_k = A p_k; partials of rt.v_k into part1.  Reads vector set a, writes set
 // b; reads state Sin, block 0 writes the advanced state to Sout.
-template <typename T>
+template <typename T, int ZC>
 __global__ __launch_bounds__(NT3) void k3_iter1(Op3<T> o, const KS3* Sin, KS3* Sout, const double* part5, int nb,
                                                 const T* ra, const T* pa, const T* va, const T* t, const T* rt,
                                                 T* rb, T* pb, T* vb, T* x, double* part1) {
@@ -611,7 +611,7 @@ __global__ __launch_bounds__(NT3) void k3_iter1(Op3<T> o, const KS3* Sin, KS3* S
   // The node plane's r, p, v, t are read once: the operand p_k is combined
   // from them for the stencil, and the tile's own nodes keep them in LDS for
   // the updates.  Node operands one step ahead, over 24-plane chunks.
-  march3<T, 1, 2, false, true, kZ1<T>, true>(
+  march3<T, 1, 2, false, true, ZC, true>(
       o, Iter1In<T>{va, ra, pa, t, al, om, be}, [&](long g) { return Ops{rt[g], x[g]}; },
       [&](long g, T y, T pn, const Ops& e, const typename Iter1In<T>::Raw& w, double(&a)[1]) {
         const T s = w.r - al * w.v;
@@ -630,7 +630,7 @@ __global__ __launch_bounds__(NT3) void k3_iter1(Op3<T> o, const KS3* Sin, KS3* S
 // rt.t into part5.  Reads state Sin, block 0 writes the advanced state to
 // Sout.  Six waves per SIMD keep three marching blocks on a CU (all 765
 // blocks of a 257x129x129 launch resident at once): at most 80 VGPRs.
-template <typename T>
+template <typename T, int ZC>
 __global__ __launch_bounds__(NT3) __attribute__((amdgpu_waves_per_eu(6))) void k3_iter2(
     Op3<T> o, const KS3* Sin, KS3* Sout, const double* part1, int nb, const T* r, const T* v, const T* rt, T* t,
     double* part5) {
@@ -648,7 +648,7 @@ __global__ __launch_bounds__(NT3) __attribute__((amdgpu_waves_per_eu(6))) void k
   const T al = (T)k.alpha;
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
   // FP64: five FP64 accumulators; its step loads stay where they are used
-  march3<T, 5, sizeof(T) == 4 ? 2 : 0, true>(
+  march3<T, 5, sizeof(T) == 4 ? 2 : 0, true, false, ZC>(
       o, [&](long g) { return r[g] - al * v[g]; }, [&](long g) { return rt[g]; },
       [&](long g, T y, T s, T rtg, double(&a)[5]) {
         t[g] = y;
@@ -796,6 +796,7 @@ int dalloc3(pb_op3d* op, T** p, long count) {
   return PB_OK;
 }
 
+const dim3 kBlk3(X3, Y3);
 dim3 march_grid(const pb_op3d* op, int zc = Z3) {
   return dim3(ceil_div(op->g.nx, X3), ceil_div(op->g.ny, Y3), ceil_div(op->g.nz, zc));
 }
@@ -813,8 +814,46 @@ int march_check(const pb_op3d* op, const dim3& grd, int zc) {
                    grd.x, grd.y, grd.z, op->g.nx, op->g.ny, op->g.nz, zc);
   return PB_OK;
 }
+
+// z planes per block of the two solver launches.  Long chunks read fewer halo
+// planes and suit grids that fill the chip.  On smaller grids a launch is bound
+// by its blocks' march, one plane after the other, and short chunks divide
+// that march while their blocks still run at once: 2 planes up to a block per
+// CU, 4 up to 2.25, 8 up to the blocks a CU holds (``resident``).  FP64 launch 1
+// + 2, us, with 24/16-, 8- and 4-plane chunks: 33x17x17 58 / 34 / 23 (2 planes: 18); 150x75x67
+// (30 tiles) 86 / 55 / 37; 220x78x55 (40 tiles) 87 / 57 / 50; 257x129x65 (85
+// tiles) 94 / 84 / 91, launch 1 47 / 52 / 54.
+inline int chunk_of(const pb_op3d* op, int resident, int full) {
+  const int cu = op->ctx->n_cu;
+  if (march_blocks(op, 2) <= cu) return 2;
+  if (4 * march_blocks(op, 4) <= 9 * cu) return 4;
+  return march_blocks(op, 8) <= resident * cu ? 8 : full;
+}
+template <typename T>
+int chunk1(const pb_op3d* op) {
+  return chunk_of(op, sizeof(T) == 8 ? 2 : 3, kZ1<T>);
+}
+inline int chunk2(const pb_op3d* op) { return chunk_of(op, 3, Z3); }
+
+template <typename T, class... A>
+void launch_iter1(const pb_op3d* op, hipStream_t s, A... args) {
+  const int zc = chunk1<T>(op);
+  const dim3 g = march_grid(op, zc);
+  if (zc == 2) hipLaunchKernelGGL((k3_iter1<T, 2>), g, kBlk3, 0, s, args...);
+  else if (zc == 4) hipLaunchKernelGGL((k3_iter1<T, 4>), g, kBlk3, 0, s, args...);
+  else if (zc == 8) hipLaunchKernelGGL((k3_iter1<T, 8>), g, kBlk3, 0, s, args...);
+  else hipLaunchKernelGGL((k3_iter1<T, kZ1<T>>), g, kBlk3, 0, s, args...);
+}
+template <typename T, class... A>
+void launch_iter2(const pb_op3d* op, hipStream_t s, A... args) {
+  const int zc = chunk2(op);
+  const dim3 g = march_grid(op, zc);
+  if (zc == 2) hipLaunchKernelGGL((k3_iter2<T, 2>), g, kBlk3, 0, s, args...);
+  else if (zc == 4) hipLaunchKernelGGL((k3_iter2<T, 4>), g, kBlk3, 0, s, args...);
+  else if (zc == 8) hipLaunchKernelGGL((k3_iter2<T, 8>), g, kBlk3, 0, s, args...);
+  else hipLaunchKernelGGL((k3_iter2<T, Z3>), g, kBlk3, 0, s, args...);
+}
 dim3 elem_grid3(long n) { return dim3((unsigned)std::min<long>((n + 255) / 256, 4096)); }
-const dim3 kBlk3(X3, Y3);
 
 template <typename T>
 Op3<T> op3(const pb_op3d* op);
@@ -883,12 +922,8 @@ int krylov3(pb_op3d* op, const T* b, double tol, int maxiter, int legacy, int ch
   const int P = Prec<T>::k;
   const long n = op->n;
   const Op3<T> o = op3<T>(op);
-  const dim3 mg = march_grid(op);
-  const int nbm = march_blocks(op);   // launch 2's blocks (five-dot records)
-  const dim3 mg1 = march_grid(op, kZ1<T>);
-  const int nb1 = march_blocks(op, kZ1<T>);   // launch 1's blocks (r~.v records)
-  if (int rc = march_check(op, mg, Z3)) return rc;       // launch 2 marches Z3-plane chunks
-  if (int rc = march_check(op, mg1, kZ1<T>)) return rc;  // launch 1 marches kZ1<T>-plane chunks
+  const int nbm = march_blocks(op, chunk2(op));      // launch 2's blocks (five-dot records)
+  const int nb1 = march_blocks(op, chunk1<T>(op));   // launch 1's blocks (r~.v records)
   const dim3 eg = elem_grid3(n);
   T* t = (T*)op->t[P];
   T* rt = (T*)op->rt[P];
@@ -910,10 +945,10 @@ int krylov3(pb_op3d* op, const T* b, double tol, int maxiter, int legacy, int ch
     for (int c = 0; c < chunk; ++c) {
       const long it = it0 + c + 1;
       const int a = (int)((it - 1) & 1), bset = (int)(it & 1);
-      hipLaunchKernelGGL(k3_iter1<T>, mg1, kBlk3, 0, s, o, (const KS3*)S0, S1, (const double*)op->part, nbm,
+      launch_iter1<T>(op, s, o, (const KS3*)S0, S1, (const double*)op->part, nbm,
                          (const T*)op->r[P][a], (const T*)op->p[P][a], (const T*)op->v[P][a], (const T*)t,
                          (const T*)rt, (T*)op->r[P][bset], (T*)op->p[P][bset], (T*)op->v[P][bset], x, op->part1);
-      hipLaunchKernelGGL(k3_iter2<T>, mg, kBlk3, 0, s, o, (const KS3*)S1, S0, (const double*)op->part1, nb1,
+      launch_iter2<T>(op, s, o, (const KS3*)S1, S0, (const double*)op->part1, nb1,
                          (const T*)op->r[P][bset], (const T*)op->v[P][bset], (const T*)rt, t, op->part);
     }
     hipLaunchKernelGGL(k3_fold, dim3(1), dim3(NRT), 0, s, S0, (const double*)op->part, nbm);
@@ -1176,8 +1211,6 @@ extern "C" int pb_op3d_time_kernel(pb_op3d* op, int kernel, int precision, int r
   const dim3 eg = elem_grid3(n), mg = march_grid(op);
   const int P = precision == PB_F64 ? 0 : 1;
   if ((rc = march_check(op, mg, Z3))) return rc;
-  if ((rc = march_check(op, march_grid(op, P == 0 ? kZ1<double> : kZ1<float>), P == 0 ? kZ1<double> : kZ1<float>)))
-    return rc;
   // vectors r, p, v, t, rt, x of both sets hold a constant pattern; the state
   // carries small fixed scalars so repeated launches stay finite
   if (P == 0) {
@@ -1193,7 +1226,7 @@ extern "C" int pb_op3d_time_kernel(pb_op3d* op, int kernel, int precision, int r
   // (1, 0.5, 1, 1, 0.5) per block: omega 0.5, beta 1 with rho = 0.75 nb;
   // launch 2 folds r~.v records of 1: alpha = rho / nb.  The solve keeps
   // running (atol 0) and every value stays finite.
-  const int nbm = march_blocks(op);
+  const int nbm = std::max(march_blocks(op, chunk2(op)), march_blocks(op, P == 0 ? chunk1<double>(op) : chunk1<float>(op)));
   KS3 k{};
   k.rho = 0.75 * nbm;
   k.alpha = 0.5;
@@ -1222,28 +1255,26 @@ extern "C" int pb_op3d_time_kernel(pb_op3d* op, int kernel, int precision, int r
                            (float*)op->v[1][1]);
     } else if (kernel == 1) {
       if (P == 0)
-        hipLaunchKernelGGL(k3_iter1<double>, march_grid(op, kZ1<double>), kBlk3, 0, s, op3<double>(op),
-                           (const KS3*)op->st, op->st + 1,
+        launch_iter1<double>(op, s, op3<double>(op), (const KS3*)op->st, op->st + 1,
                            (const double*)op->part, nbm, (const double*)op->r[0][0], (const double*)op->p[0][0],
                            (const double*)op->v[0][0], (const double*)op->t[0], (const double*)op->rt[0],
                            (double*)op->r[0][1], (double*)op->p[0][1], (double*)op->v[0][1], (double*)op->x[0],
                            op->part1);
       else
-        hipLaunchKernelGGL(k3_iter1<float>, march_grid(op, kZ1<float>), kBlk3, 0, s, op3<float>(op),
-                           (const KS3*)op->st, op->st + 1,
+        launch_iter1<float>(op, s, op3<float>(op), (const KS3*)op->st, op->st + 1,
                            (const double*)op->part, nbm, (const float*)op->r[1][0], (const float*)op->p[1][0],
                            (const float*)op->v[1][0], (const float*)op->t[1], (const float*)op->rt[1],
                            (float*)op->r[1][1], (float*)op->p[1][1], (float*)op->v[1][1], (float*)op->x[1],
                            op->part1);
     } else {   // reads part1's records and writes its own five-dot records to part
       if (P == 0)
-        hipLaunchKernelGGL(k3_iter2<double>, mg, kBlk3, 0, s, op3<double>(op), (const KS3*)op->st, op->st + 1,
-                           (const double*)op->part1, march_blocks(op, kZ1<double>), (const double*)op->r[0][0],
+        launch_iter2<double>(op, s, op3<double>(op), (const KS3*)op->st, op->st + 1,
+                         (const double*)op->part1, march_blocks(op, chunk1<double>(op)), (const double*)op->r[0][0],
                            (const double*)op->v[0][0],
                            (const double*)op->rt[0], (double*)op->t[0], op->part);
       else
-        hipLaunchKernelGGL(k3_iter2<float>, mg, kBlk3, 0, s, op3<float>(op), (const KS3*)op->st, op->st + 1,
-                           (const double*)op->part1, march_blocks(op, kZ1<float>), (const float*)op->r[1][0],
+        launch_iter2<float>(op, s, op3<float>(op), (const KS3*)op->st, op->st + 1,
+                         (const double*)op->part1, march_blocks(op, chunk1<float>(op)), (const float*)op->r[1][0],
                            (const float*)op->v[1][0],
                            (const float*)op->rt[1], (float*)op->t[1], op->part);
     }
