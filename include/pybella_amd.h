@@ -33,6 +33,8 @@
 #ifndef PYBELLA_AMD_H
 #define PYBELLA_AMD_H
 
+#include <stdint.h>
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -255,6 +257,10 @@ int pb_correction_nodes(pb_ctx* ctx, const pb_grid2d* grid, const pb_phys* phys,
 int pb_scatter_update_p2(pb_ctx* ctx, const pb_grid2d* grid, const double* x,
                          double* p2_full, double* p2_nodes);
 
+/* dst[k][0 .. n[k]) = src[k][0 .. n[k]) for count (1 to 8) device arrays in one
+ * launch; the arrays do not overlap.  The state copies of the time step. */
+int pb_copy_fields(pb_ctx* ctx, int count, const double* const* src, double* const* dst, const int64_t* n);
+
 /* ---- explicit parts of the time step ----
  * Face-flux arrays: x faces (ny+3) x (nx+4) in [y][face] (the reference's
  * flux[0] as it lies), y faces (ny+4) x (nx+3) in [face][x] (the transpose of
@@ -392,9 +398,10 @@ int pb_op2d_mg_features(pb_op2d* op, float* f1, float* f2);
  * No reference counterpart: the reference solves members one after the other
  * (src/__main__.py:223-254, each through second_projection.py:230).  A batch
  * holds distinct assembled operators (one per member, each with its own tile
- * height); a solve captures one chunk of iterations of every member as a
- * single hipGraph (one branch per member) and replays it until all members
- * are final.  Per member the iterates equal a single solve's. */
+ * height); members whose tiles fit on the chip together run as one launch,
+ * the rest as chunks of iterations of every member in one hipGraph, replayed
+ * until all members are final.  Per member the iterates equal a single
+ * solve's. */
 int pb_batch_create(pb_ctx* ctx, pb_op2d* const* ops, int count, pb_batch** out);
 int pb_batch_destroy(pb_batch* batch);
 /* b[m], x[m]: device FP64 Krylov vectors of member m.  Modes

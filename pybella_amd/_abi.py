@@ -108,6 +108,7 @@ SIGNATURES = {
     "pb_divergence_nodes": (I, [VP, C.POINTER(Grid2D), D, VP, VP, VP, VP, VP, VP]),
     "pb_correction_nodes": (I, [VP, C.POINTER(Grid2D), C.POINTER(Phys), D, D, VP, VP, VP, VP,
                                 VP, VP, VP, VP, VP, VP]),
+    "pb_copy_fields": (I, [VP, I, C.POINTER(VP), C.POINTER(VP), C.POINTER(C.c_int64)]),
     "pb_scatter_update_p2": (I, [VP, C.POINTER(Grid2D), VP, VP, VP]),
     "pb_nn_create": (I, [VP, C.c_ulonglong, C.POINTER(VP)]),
     "pb_nn_destroy": (I, [VP]),

@@ -261,6 +261,15 @@ def _nonhydrostasy(ud, step):
     return float(ud.is_nonhydrostatic)
 
 
+def copy_fields(M: DeviceModel, src, dst):
+    """Contiguous device arrays copied in one launch on the model's stream."""
+    src, dst = list(src), list(dst)
+    k = len(src)
+    n = (C.c_int64 * k)(*[t.numel() for t in src])
+    M.ctx.check(M.ctx.lib.pb_copy_fields(M.ctx.h, k, (C.c_void_p * k)(*[t.data_ptr() for t in src]),
+                                         (C.c_void_p * k)(*[t.data_ptr() for t in dst]), n), "pb_copy_fields")
+
+
 def step_begin(M: DeviceModel, t, tout, step_no, window_step):
     """time_update.py:121-250 up to the first projection's solve: ghost
     cells, dt, the regime functions, Sol0, the advective fluxes, the RK half
@@ -277,12 +286,10 @@ def step_begin(M: DeviceModel, t, tout, step_no, window_step):
             dt = 21.69 / ud.t_ref
     ud.compressibility = _compressibility(ud, window_step)
     ud.nonhydrostasy = _nonhydrostasy(ud, window_step)
-    for d, s in zip(M.sol0.f.values(), F.values()):
-        d.copy_(s)
+    copy_fields(M, [*F.values(), M.p2n], [*M.sol0.f.values(), M.p2n0])   # p2n is not touched before p2n0's use
     recompute_advective_fluxes(M)
     if getattr(ud, "do_advection", True):
         advect_rk(M, 0.5 * dt, step_no % 2)
-    M.p2n0.copy_(M.p2n)
     euler_backward_non_advective_expl_part(M, 0.5 * dt)
     return dt, cfl, cfl_ac, project_prepare(M, 0.5 * dt, with_sol0=(ud.is_compressible == 0))
 
@@ -296,20 +303,11 @@ def step_middle(M: DeviceModel, dt, step_no, pr, x):
     F = M.sol.f
     sp._project_update(pr, x)
     recompute_advective_fluxes(M)
-    for d, s in zip(M.half, F.values()):
-        d.copy_(s)
-    M.p2_half.copy_(M.p2n)
-    if ud.is_compressible == 1 and ud.is_nonhydrostatic == 1:
-        M.p2n.copy_(M.p2n0)
-        for d, s in zip(F.values(), M.sol0.f.values()):
-            d.copy_(s)
-    elif ud.is_nonhydrostatic == 0:
-        for d, s in zip(F.values(), M.sol0.f.values()):
-            d.copy_(s)
-        M.p2n.copy_(M.p2n0)
+    copy_fields(M, [*F.values(), M.p2n], [*M.half, M.p2_half])
+    if ud.is_nonhydrostatic == 0 or (ud.is_compressible == 1 and ud.is_nonhydrostatic == 1):
+        copy_fields(M, [*M.sol0.f.values(), M.p2n0], [*F.values(), M.p2n])
     elif ud.is_compressible == 0:
-        for d, s in zip(F.values(), M.sol0.f.values()):
-            d.copy_(s)
+        copy_fields(M, M.sol0.f.values(), F.values())
     euler_forward_non_advective(M, 0.5 * dt)
     if getattr(ud, "do_advection", True):
         advect(M, dt, step_no % 2)
