@@ -798,7 +798,10 @@ int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int 
   }
   for (int m = 0; m < count; ++m)   // tags of a run: three per iteration, far from wrapping
     if (jobs[m].maxiter > (1 << 28)) return 0;
-  // one launch per kind of kernel, the members with the most tiles first
+  // Launches of one kind of kernel each, the members with the most tiles first,
+  // and never more tiles in one launch than are resident at once: blocks go to
+  // the XCDs in turn, so a member that had to wait for slots of another could
+  // get all of them on some XCDs and too few on others, and wait for good.
   std::vector<int> order(count);
   for (int m = 0; m < count; ++m) order[m] = m;
   auto kind = [&](int m) {
@@ -814,15 +817,22 @@ int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int 
   });
   // check the room of every launch before the first one
   int need = 0;
+  struct Span {
+    int f, e;
+    ResKernel<T> fn;
+  };
+  std::vector<Span> spans;
   for (int f = 0; f < count;) {
-    int e = f, total = 0;
-    while (e < count && kind(order[e]) == kind(order[f])) total += tiles(order[e++]);
     const pb_op2d* op = jobs[order[f]].op;
     const ResKernel<T> fn = pick<T>(op->ry, op->cross, op->center, exact, tiles(order[f]) > 2 * ctx->n_cu);
     int occ = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)fn, NTHR, 0) != hipSuccess || occ < 1) return 0;
-    if (tiles(order[f]) > std::min(occ * ctx->n_cu, kMaxPerLane * NTHR)) return 0;
+    const int slots = occ * ctx->n_cu;
+    if (tiles(order[f]) > std::min(slots, kMaxPerLane * NTHR)) return 0;
+    int e = f, total = 0;
+    while (e < count && kind(order[e]) == kind(order[f]) && total + tiles(order[e]) <= slots) total += tiles(order[e++]);
     need = std::max(need, std::min(ctx->n_cu, ceil_div(total, occ)));
+    spans.push_back(Span{f, e, fn});
     f = e;
   }
   Room room;
@@ -836,6 +846,7 @@ int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int 
   ResOut* const dres = (ResOut*)((char*)rec.dev + tab_bytes);
   std::vector<int> total;
   for (int k = 0; k < count; ++k) {
+    if (total.size() < spans.size() && k == spans[total.size()].f) total.push_back(0);
     const ResJob<T>& J = jobs[order[k]];
     pb_op2d* op = J.op;
     Resident* R = resident_of(op);
@@ -847,8 +858,6 @@ int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int 
       R->cleared = true;
       R->epoch = 0;
     }
-    const bool first = k == 0 || kind(order[k]) != kind(order[k - 1]);
-    if (first) total.push_back(0);
     const dim3 g = stencil_grid(op, op->ry);
     RMember<T>& M = tab[k];
     M.op = opdev<T>(op);
@@ -876,16 +885,11 @@ int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int 
     R->epoch += span;
   }
   PB_HIP(ctx, hipMemcpyAsync(rec.dev, rec.host, tab_bytes + out_bytes, hipMemcpyHostToDevice, s));
-  for (int f = 0, l = 0; f < count; ++l) {
-    int e = f;
-    while (e < count && kind(order[e]) == kind(order[f])) ++e;
-    const pb_op2d* op = jobs[order[f]].op;
-    const ResKernel<T> fn = pick<T>(op->ry, op->cross, op->center, exact, tiles(order[f]) > 2 * ctx->n_cu);
-    hipLaunchKernelGGL(fn, dim3((unsigned)total[l]), dim3(TX, TYT), 0, s, (const RMember<T>*)(dtab + f), e - f,
-                       rec.ticket, rec.ticket_next);
+  for (size_t l = 0; l < spans.size(); ++l) {
+    hipLaunchKernelGGL(spans[l].fn, dim3((unsigned)total[l]), dim3(TX, TYT), 0, s, (const RMember<T>*)(dtab + spans[l].f),
+                       spans[l].e - spans[l].f, rec.ticket, rec.ticket_next);
     PB_LAUNCH_CHECK(ctx);
     rec.ticket_next += (unsigned)total[l];
-    f = e;
   }
   PB_HIP(ctx, hipMemcpyAsync(res, dres, out_bytes, hipMemcpyDeviceToHost, s));
   PB_HIP(ctx, hipStreamSynchronize(s));
