@@ -1,6 +1,6 @@
 """Batched uneven 2D solves (pb_batch_*): many assembled operators, possibly
-of different grid sizes, solved together: one launch for members whose tiles
-fit on the chip, else one hipGraph per chunk of iterations.  No reference counterpart: the reference
+of different grid sizes, solved together: resident launches for members whose
+tiles fit on the chip, else one hipGraph per chunk of iterations.  No reference counterpart: the reference
 solves ensemble members one after the other (src/__main__.py:223-254)."""
 from __future__ import annotations
 

@@ -6,8 +6,8 @@ whole time-step driver (src/__main__.py:223-254: ``dis_time_update.do`` per
 member).  Here every member keeps its own device state and operator, the
 members advance in lockstep (each with its own dt and time, exactly as its own
 ``do`` would), and at each of a step's two projections the solves of all
-members run as one batched solve (pb_batch_solve: one launch for members that
-fit on the chip, else one hipGraph per chunk of iterations).  Every member's
+members run as one batched solve (pb_batch_solve: resident launches for members
+that fit on the chip, else one hipGraph per chunk of iterations).  Every member's
 result equals its single-member GPU step with the same solver mode, bit for bit.
 """
 from __future__ import annotations
