@@ -25,6 +25,8 @@ using namespace pb2d;
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4), may_alias));   // 16 bytes of anything
+typedef int i32any __attribute__((may_alias));
 // LDS of a convolution block's weight tile: 16 NT rows x (cin + 4); the
 // launches keep 16 NT cin <= 8192 (checked on the host)
 constexpr int kConvWsh = 8192 + 64 * 4;
@@ -287,116 +289,153 @@ __global__ __launch_bounds__(256) void k_conv3x3_small(const bf16* __restrict__ 
 
 // ---------------------------------------------------------------------------
 // weight and bias gradient: dW[tap][ci][co] = sum_p in[p + off(tap)][ci]
-// dz[p][co], db[co] = sum_p dz[p][co].  Block (co tile, ci tile) x pixel chunk;
-// wave-strided 16-pixel steps; MFMA with A[co][pixel] = dz, B[pixel][ci] =
-// shifted input.  Partials per chunk.
-// A step is bound by the latency of its 40 two-byte loads: they are all
-// unconditional (clamped index, then select), so they go out together, the
-// pixel's coordinates are stepped instead of divided out, and short chunks
-// (128 pixels up, see wgrad) keep ~1000 blocks in flight.  32 images of 33x65,
-// 15 layers: 74 -> 10.7 us per layer with 1024-pixel chunks, guarded loads and
-// 64-bit divisions before; the bias sums ride along (40 us per layer in two
-// launches of their own).
+// dz[p][co], db[co] = sum_p dz[p][co].
+// A weight block takes one chunk of up to ~1024 pixels, a (ci tile, co tile)
+// and a row of three taps; its 12 waves are the three taps times four shares of
+// the 16-pixel steps; MFMA with A[co][pixel] = dz, B[pixel][ci] = shifted
+// input.  Bias blocks sum three chunks of 256 pixels each, four interleaved sums
+// per channel.  k_wgrad_reduce adds the chunks in turn.  The order of every sum
+// is fixed by the shape: a share's steps in turn, the four shares pairwise, the
+// chunks in turn; the split into taps and rows touches no sum.
+// Bound by latency: read from global, a step was 40 two-byte loads and the
+// pixels' divisions.  The chunk's values come into LDS with one round of 16-byte
+// loads, with a byte per pixel that says which taps stay inside the image, and
+// the steps read LDS.  32 images of 33x65, 15 layers, us per layer with its
+// reduction: 74 + 40 for the bias (a block per chunk and tile pair, guarded
+// two-byte loads) -> 9.1 + 5.4.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_wgrad(const bf16* __restrict__ in, int in_ctot, int in_coff, int cin,
-                                               const bf16* __restrict__ dz, int dz_ctot, int dz_coff, int cout,
-                                               int nimg, int h, int w, long chunk, float* partial, float* bpartial) {
-  __shared__ float red[4][9][16][17];
-  __shared__ float bred[4][64];
+constexpr int kWgTile = 1024;       // pixels staged at once
+constexpr int kWgThreads = 12 * 64;
+__global__ __launch_bounds__(kWgThreads) void k_wgrad(const bf16* __restrict__ in, int in_ctot, int in_coff, int cin,
+                                                      const bf16* __restrict__ dz, int dz_ctot, int dz_coff, int cout,
+                                                      int cout_v, int nimg, int h, int w, int nchunk, int chunk,
+                                                      int nbchunk, int bchunk, float* partial, float* bpartial) {
+  struct Stage {
+    bf16 a[kWgTile][16], v[kWgTile + 2][16];
+    __align__(4) unsigned char ok[kWgTile];   // 1: the row dy away is in the image, 2: so is the left, 4: the right pixel there
+  };
+  union Lds {
+    Stage st;
+    float red[4][3][16][17];
+  };
+  __shared__ __align__(16) Lds sh;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int nct = cout / 16;
-  const int cot = blockIdx.y % nct, cit = blockIdx.y / nct;
   const int npix = nimg * h * w;   // the shape allocator refuses tensors past 2^31 values
-  const int pbeg = (int)((long)blockIdx.x * chunk);
-  const int pend = (int)(pbeg + chunk < npix ? pbeg + chunk : npix);
-  const int kg = lane >> 4, l16 = lane & 15;
-  f32x4 acc[9];
-#pragma unroll
-  for (int t = 0; t < 9; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float bsum = 0.f;
-  const int dch = dz_coff + cot * 16 + l16, ich = in_coff + cit * 16 + l16;
-  int p = pbeg + wave * 16 + 4 * kg, x = p % w, y = (p / w) % h;
-  for (int p0 = pbeg + wave * 16; p0 < pend; p0 += 64) {
-    bf16x4 a, bt[9];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      int xe = x + e, ye = y;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {   // the four pixels cross three row ends at most (w = 1)
-        if (xe >= w) {
-          xe -= w;
-          ye = ye + 1 == h ? 0 : ye + 1;
-        }
-      }
-      const int pe = p + e;
-      const bool ok = pe < pend;
-      const short av = (short)dz[ok ? pe * dz_ctot + dch : 0];
-      a[e] = ok ? av : (short)0;
-#pragma unroll
-      for (int tap = 0; tap < 9; ++tap) {
-        const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-        const bool in_img = ok && (dy < 0 ? ye > 0 : dy > 0 ? ye < h - 1 : true) &&
-                            (dx < 0 ? xe > 0 : dx > 0 ? xe < w - 1 : true);
-        const short bv = (short)in[in_img ? (pe + dy * w + dx) * in_ctot + ich : 0];
-        bt[tap][e] = in_img ? bv : (short)0;
-      }
-    }
-#pragma unroll
-    for (int tap = 0; tap < 9; ++tap) acc[tap] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bt[tap], acc[tap], 0, 0, 0);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) bsum += bf2f((bf16)a[e]);
-    p += 64;
-    x += 64;
-    while (x >= w) {
-      x -= w;
-      y = y + 1 == h ? 0 : y + 1;
-    }
-  }
-  // acc[tap][e] = D[co = 4 kg + e][ci = l16]
-#pragma unroll
-  for (int tap = 0; tap < 9; ++tap)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) red[wave][tap][4 * kg + e][l16] = acc[tap][e];
-  bred[wave][lane] = bsum;
-  __syncthreads();
-  for (int k = threadIdx.x; k < 9 * 256; k += 256) {
-    const int tap = k / 256, rem = k % 256, ci = rem / 16, co = rem % 16;
-    const float s = (red[0][tap][co][ci] + red[1][tap][co][ci]) + (red[2][tap][co][ci] + red[3][tap][co][ci]);
-    // partial layout [chunk][tap][ci][co] over the padded cin x cout
-    partial[(((long)blockIdx.x * 9 + tap) * cin + cit * 16 + ci) * cout + cot * 16 + co] = s;
-  }
-  if (cit == 0 && threadIdx.x < 16) {
+  const int nct = cout / 16, nweight = nchunk * nct * (cin / 16) * 3;
+  if ((int)blockIdx.x >= nweight) {   // three bias chunks, four waves each
+    constexpr int U = 16;
+    const int c = 3 * (blockIdx.x - nweight) + wave / 4, pbeg = min(c * bchunk, npix), pend = min(pbeg + bchunk, npix);
     float s = 0.f;
-    for (int k = 0; k < 4; ++k)
-      for (int q = 0; q < 4; ++q) s += bred[k][16 * q + threadIdx.x];
-    bpartial[(long)blockIdx.x * cout + cot * 16 + threadIdx.x] = s;
+    if (lane < cout_v) {
+      const bf16* src = dz + dz_coff + lane;
+      for (int p = pbeg + wave % 4; p < pend; p += 4 * U) {
+        float v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = bf2f(src[min(p + 4 * u, npix - 1) * dz_ctot]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) s = p + 4 * u < pend ? s + v[u] : s;
+      }
+    }
+    float* const sb = &sh.red[0][0][0][0];
+    sb[threadIdx.x] = s;
+    __syncthreads();
+    if (wave % 4 == 0 && lane < cout_v && c < nbchunk) {
+      s = 0.f;
+      for (int k = 0; k < 4; ++k) s += sb[threadIdx.x + 64 * k];
+      bpartial[(long)c * 64 + lane] = s;
+    }
+    return;
+  }
+  const int bc = blockIdx.x % nchunk, bt = blockIdx.x / nchunk, row = bt % 3, tile = bt / 3;
+  const int cot = tile % nct, cit = tile / nct, dy = row - 1;
+  const int t = wave >> 2, part = wave & 3;   // the wave's tap of the row and its share of the steps
+  const int pbeg = bc * chunk, len = min(chunk, npix - pbeg);
+  const int kg = lane >> 4, l16 = lane & 15;
+  const int bit = t == 0 ? 1 : t == 1 ? 0 : 2;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < len; s0 += kWgTile) {
+    const int m = min(kWgTile, len - s0), p0 = pbeg + s0, q0 = p0 + dy * w - 1;
+    constexpr int N = (2 * (kWgTile + 2) + kWgThreads - 1) / kWgThreads;   // 16-byte halves of a pixel per thread
+    i32x4 a[N], v[N];
+    const bf16* const az = dz + dz_coff + cot * 16;
+    const bf16* const vi = in + in_coff + cit * 16;
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int k = threadIdx.x + kWgThreads * u, i = k >> 1, q = q0 + i;
+      a[u] = *(const i32x4*)(az + (i < m ? (p0 + i) * dz_ctot + (k & 1) * 8 : 0));
+      v[u] = *(const i32x4*)(vi + ((unsigned)q < (unsigned)npix && i < m + 2 ? q * in_ctot + (k & 1) * 8 : 0));
+    }
+    if (s0) __syncthreads();   // the steps have read the tile before
+    for (int i = threadIdx.x; i < kWgTile; i += kWgThreads) {
+      const int p = p0 + i, x = p % w, y = p / w % h + dy;
+      sh.st.ok[i] = (unsigned char)(i < m && y >= 0 && y < h ? 1 + (x > 0 ? 2 : 0) + (x < w - 1 ? 4 : 0) : 0);
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int k = threadIdx.x + kWgThreads * u, i = k >> 1;
+      if (i < kWgTile) ((i32x4*)sh.st.a)[k] = i < m ? a[u] : i32x4{0, 0, 0, 0};
+      if (i < m + 2) ((i32x4*)sh.st.v)[k] = v[u];
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int i0 = part * 16; i0 < m; i0 += 64) {
+      const int i = i0 + 4 * kg, f = *(const i32any*)(sh.st.ok + i) >> bit;
+      bf16x4 av, bv;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        av[e] = (short)sh.st.a[i + e][l16];
+        const short x = (short)sh.st.v[i + e + t][l16];
+        bv[e] = (f >> 8 * e & 1) ? x : (short)0;
+      }
+      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
+    }
+  }
+  __syncthreads();
+  // acc[e] = D[co = 4 kg + e][ci = l16]
+#pragma unroll
+  for (int e = 0; e < 4; ++e) sh.red[part][t][4 * kg + e][l16] = acc[e];
+  __syncthreads();
+  for (int k = threadIdx.x; k < 3 * 256; k += kWgThreads) {
+    const int tk = k / 256, rem = k % 256, ci = rem / 16, co = rem % 16;
+    const float s = (sh.red[0][tk][co][ci] + sh.red[1][tk][co][ci]) + (sh.red[2][tk][co][ci] + sh.red[3][tk][co][ci]);
+    // partial layout [chunk][tap][ci][co] over the padded cin x cout
+    partial[(((long)bc * 9 + row * 3 + tk) * cin + cit * 16 + ci) * cout + cot * 16 + co] = s;
   }
 }
 
-// sum the chunk partials into the master gradients [9][cin_v][cout_v] and
-// [cout_v] (true dims): 64 values per block, 16 waves sharing the chunks
-constexpr int kRedWaves = 16;
+// sum the chunk partials, chunk after chunk, into the master gradients
+// [9][cin_v][cout_v] and [cout_v] (true dims): 64 values per block, whose 16
+// waves stage kRedTile chunks at a time for the wave that adds them
+constexpr int kRedWaves = 16, kRedTile = 128;
 __global__ __launch_bounds__(64 * kRedWaves) void k_wgrad_reduce(const float* __restrict__ partial,
                                                                  const float* __restrict__ bpartial, int nchunk,
-                                                                 int cin, int cout, int cin_v, int cout_v, float* g,
-                                                                 float* gb) {
-  __shared__ float sh[kRedWaves][64];
+                                                                 int nbchunk, int cin, int cout, int cin_v, int cout_v,
+                                                                 float* g, float* gb) {
+  __shared__ float sh[kRedTile][64];
   const int n = 9 * cin_v * cout_v, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int k = blockIdx.x * 64 + lane;
   const bool ok = k < n + cout_v;
   const int co = k < n ? k % cout_v : k - n, t1 = k / cout_v;
   const float* src = !ok ? partial : k < n ? partial + ((long)(t1 / cin_v) * cin + t1 % cin_v) * cout + co : bpartial + co;
-  const long step = !ok ? 0 : k < n ? 9L * cin * cout : cout;
+  const long step = !ok ? 0 : k < n ? 9L * cin * cout : 64;
+  const int cnt = !ok ? 0 : k < n ? nchunk : nbchunk;
+  const int most = (blockIdx.x + 1) * 64 > n ? max(nchunk, nbchunk) : nchunk;
   float s = 0.f;
-#pragma unroll 8
-  for (int c = wave; c < nchunk; c += kRedWaves) s += src[c * step];
-  sh[wave][lane] = s;
-  __syncthreads();
-  if (wave == 0 && ok) {
-    s = 0.f;
-    for (int q = 0; q < kRedWaves; ++q) s += sh[q][lane];
-    (k < n ? g[k] : gb[co]) = s;
+  for (int c0 = 0; c0 < most; c0 += kRedTile) {
+    float v[kRedTile / kRedWaves];
+#pragma unroll
+    for (int u = 0; u < kRedTile / kRedWaves; ++u) v[u] = src[max(0, min(c0 + u * kRedWaves + wave, cnt - 1)) * step];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kRedTile / kRedWaves; ++u) sh[u * kRedWaves + wave][lane] = v[u];
+    __syncthreads();
+    if (wave == 0) {
+      const int m = min(kRedTile, cnt - c0);
+#pragma unroll 16
+      for (int c = 0; c < m; ++c) s += sh[c][lane];
+    }
   }
+  if (wave == 0 && ok) (k < n ? g[k] : gb[co]) = s;
 }
 
 // dz *= gelu'(pre) on a view
@@ -984,17 +1023,19 @@ int wgrad(pb_nn* nn, Acts* a, int l, int level, const bf16* in, int in_ct, int i
   const long npix = (long)a->nimg * a->lv[level].h * a->lv[level].w;
   const int h = a->lv[level].h, w = a->lv[level].w;
   const int ntiles = (cin_p / 16) * (cout_p / 16);
-  // chunks of 128 pixels up to ~1000 blocks, of 1024 pixels beyond
-  int nchunk = (int)std::max<long>(std::min<long>(1024 / ntiles, (npix + 127) / 128), (npix + 1023) / 1024);
-  nchunk = std::max(1, std::min(nchunk, 2048 / ntiles));
+  int nchunk = (int)std::max<long>(1, std::min<long>(2048 / ntiles, (npix + 1023) / 1024));
   const long chunk = (npix + nchunk - 1) / nchunk;
   nchunk = (int)((npix + chunk - 1) / chunk);
+  int nbchunk = (int)std::min<long>(1024, (npix + 255) / 256);
+  const long bchunk = (npix + nbchunk - 1) / nbchunk;
+  nbchunk = (int)((npix + bchunk - 1) / bchunk);
   const long need = (long)nchunk * 9 * cin_p * cout_p;
   if (need > nn->wpart_cap) return pb_fail(nn->ctx, PB_ERR_STATE, "wgrad partial buffer too small");
-  hipLaunchKernelGGL(k_wgrad, dim3(nchunk, ntiles), dim3(256), 0, s, in, in_ct, in_co, cin_p, dz, dz_ct, dz_co, cout_p,
-                     a->nimg, h, w, chunk, nn->wpart, nn->bpart);
+  hipLaunchKernelGGL(k_wgrad, dim3(3 * nchunk * ntiles + ceil_div(nbchunk, 3)), dim3(kWgThreads), 0, s, in, in_ct, in_co, cin_p, dz, dz_ct,
+                     dz_co, cout_p, L.cout_v, a->nimg, h, w, nchunk, (int)chunk, nbchunk, (int)bchunk, nn->wpart,
+                     nn->bpart);
   hipLaunchKernelGGL(k_wgrad_reduce, dim3(ceil_div(9 * L.cin_v * L.cout_v + L.cout_v, 64)), dim3(64 * kRedWaves), 0, s,
-                     (const float*)nn->wpart, (const float*)nn->bpart, nchunk, cin_p, cout_p, L.cin_v, L.cout_v,
+                     (const float*)nn->wpart, (const float*)nn->bpart, nchunk, nbchunk, cin_p, cout_p, L.cin_v, L.cout_v,
                      nn->grads + nn->woff[l], nn->grads + nn->boff[l]);
   return PB_OK;
 }
@@ -1319,7 +1360,7 @@ extern "C" int pb_nn_create(pb_ctx* ctx, unsigned long long seed, pb_nn** out) {
   }
   nn->wpart_cap = 2048L * 9 * 16 * 16 + 9L * 128 * 64;
   rc |= nn_malloc(nn, nn->allocs, &nn->wpart, nn->wpart_cap);
-  rc |= nn_malloc(nn, nn->allocs, &nn->bpart, 2048L * 64);
+  rc |= nn_malloc(nn, nn->allocs, &nn->bpart, 1024L * 64);
   if (rc) {
     pb_nn_destroy(nn);
     return PB_ERR_HIP;
