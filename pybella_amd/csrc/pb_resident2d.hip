@@ -198,6 +198,11 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
     sid = (int)(atomicAdd(ticket, 1u) - ticket0);
   }
   for (int k = tid; k < (TY + 2 + RY) * (TX + 2); k += NTHR) sp[k] = T(0);
+  // A class of records no tile belongs to adds zero.  Cleared here, before the
+  // barrier, and not in the exchanges: which classes are written depends on the
+  // tile count alone, and from 65 to 96 tiles other waves write theirs with no
+  // barrier in between.
+  if (tid < 5 * NW) ssum[tid] = 0.0;
   __syncthreads();
   const int blk = __builtin_amdgcn_readfirstlane(sid);
   int m = 0;
@@ -385,7 +390,6 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
 #pragma unroll
         for (int w = 0; w < NW; ++w) own += sred[lane * NW + w];
       }
-      if (lane < NV * NW) ssum[lane] = 0.0;
       if (nb == 1) {
         if (lane < NV) ssum[lane * NW] = own;
       } else if (lane < NV) {

@@ -55,6 +55,22 @@ def test_resident_equals_launches(nx, ny, ry, kind, mode):
     op.close()
 
 
+@pytest.mark.parametrize("mode", ["f64fast", "f64"])
+@pytest.mark.parametrize("nx,ny,tiles", [(509, 125, 64), (301, 205, 65), (509, 140, 72), (301, 301, 95),
+                                         (509, 190, 96), (570, 170, 99)])
+def test_class_sums_at_each_way_of_summing(nx, ny, tiles, mode):
+    """Tile counts at the ends of each way of summing the records: one wave up
+    to 64, two waves writing class sums of their own from 65 to 96, class sums
+    formed by other blocks above."""
+    print(f"case resident {tiles} tiles {mode}", flush=True)
+    assert -(-nx // 64) * -(-ny // 16) == tiles
+    op, b = _system(nx, ny, "coriolis")
+    op.set_tile(4)
+    for k in (1, 3, 60):
+        _same(op, b, tol=1e-30, maxiter=k, mode=mode)
+    op.close()
+
+
 def test_more_tiles_than_two_per_unit_and_guess():
     """561 tiles of 16 rows (three blocks on some compute units), a given
     guess, a zero right-hand side and an exact one."""
