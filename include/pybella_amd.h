@@ -44,6 +44,18 @@ extern "C" {
 #define PB_ERR_HIP (-2)
 #define PB_ERR_STATE (-3)
 
+/* pb_ctx_set_resident */
+#define PB_RESIDENT_OFF 0      /* Krylov runs by launches per phase              */
+#define PB_RESIDENT_ON 1       /* on the chip in one launch, where they fit      */
+#define PB_RESIDENT_GIVE_UP 2  /* as ON, each run then given up and repeated by
+                                  launches: the way a wait that ran out goes     */
+/* pb_ctx_resident_runs */
+#define PB_RESIDENT_RUNS 0      /* Krylov runs that stayed on the chip           */
+#define PB_RESIDENT_LAUNCHES 1  /* the launches they took (a batch shares them)  */
+#define PB_RESIDENT_DECLINED 2  /* runs by launches per phase                    */
+#define PB_RESIDENT_GIVEN_UP 3  /* runs whose wait ran out, repeated by launches */
+#define PB_RESIDENT_COUNTS 4
+
 #define PB_BC_PERIODIC 0
 #define PB_BC_WALL 1
 
@@ -145,6 +157,12 @@ int pb_ctx_destroy(pb_ctx* ctx);
  * uses a non-blocking stream of its own until this is called. */
 int pb_ctx_set_stream(pb_ctx* ctx, void* hip_stream);
 int pb_ctx_synchronize(pb_ctx* ctx);
+/* Whether the context's BiCGStab runs may stay on the chip (one launch per run,
+ * PB_RESIDENT_ON at first); results are the same bit for bit.  Also ends the
+ * pause after runs that were given up. */
+int pb_ctx_set_resident(pb_ctx* ctx, int mode);
+/* counts[PB_RESIDENT_COUNTS] since the context was made */
+int pb_ctx_resident_runs(const pb_ctx* ctx, int64_t* counts);
 const char* pb_last_error(const pb_ctx* ctx);
 
 /* cell ghost fill: wrap / mirror in x, hydrostatic images in y (gravity axis).

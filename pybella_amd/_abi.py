@@ -20,6 +20,9 @@ PB_SOLVE_MIXED = 1
 PB_SOLVE_NN = 2
 PB_SOLVE_F64_FAST = 3
 PB_SOLVE_F64_FUSED = 4
+PB_RESIDENT_OFF = 0
+PB_RESIDENT_ON = 1
+PB_RESIDENT_GIVE_UP = 2
 
 
 class Grid2D(C.Structure):
@@ -82,6 +85,8 @@ SIGNATURES = {
     "pb_ctx_destroy": (I, [VP]),
     "pb_ctx_set_stream": (I, [VP, VP]),
     "pb_ctx_synchronize": (I, [VP]),
+    "pb_ctx_set_resident": (I, [VP, I]),
+    "pb_ctx_resident_runs": (I, [VP, C.c_int64 * 4]),
     "pb_last_error": (C.c_char_p, [VP]),
     "pb_bc_cells": (I, [VP, C.POINTER(Grid2D), C.POINTER(Phys), VP * 6, VP]),
     "pb_ghostnodes": (I, [VP, C.POINTER(Grid2D), VP]),
@@ -179,6 +184,17 @@ class Context:
 
     def synchronize(self):
         self.check(self.lib.pb_ctx_synchronize(self.h), "pb_ctx_synchronize")
+
+    def set_resident(self, mode):
+        """Whether Krylov runs may stay on the chip (PB_RESIDENT_*)."""
+        self.check(self.lib.pb_ctx_set_resident(self.h, mode), "pb_ctx_set_resident")
+
+    def resident_runs(self):
+        """Krylov runs so far: on the chip, their launches, declined (run by
+        launches per phase), given up (repeated by launches per phase)."""
+        n = (C.c_int64 * 4)()
+        self.check(self.lib.pb_ctx_resident_runs(self.h, n), "pb_ctx_resident_runs")
+        return dict(zip(("runs", "launches", "declined", "given_up"), n))
 
     def close(self):
         if getattr(self, "h", None):

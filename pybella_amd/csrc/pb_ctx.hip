@@ -89,4 +89,19 @@ extern "C" int pb_ctx_synchronize(pb_ctx* ctx) {
   return PB_OK;
 }
 
+extern "C" int pb_ctx_set_resident(pb_ctx* ctx, int mode) {
+  if (!ctx) return PB_ERR_ARG;
+  if (mode != PB_RESIDENT_OFF && mode != PB_RESIDENT_ON && mode != PB_RESIDENT_GIVE_UP)
+    return pb_fail(ctx, PB_ERR_ARG, "pb_ctx_set_resident: mode %d", mode);
+  ctx->resident_mode.store(mode);
+  ctx->resident_skip.store(0);
+  return PB_OK;
+}
+
+extern "C" int pb_ctx_resident_runs(const pb_ctx* ctx, int64_t* counts) {
+  if (!ctx || !counts) return PB_ERR_ARG;
+  for (int k = 0; k < PB_RESIDENT_COUNTS; ++k) counts[k] = ctx->resident_count[k].load();
+  return PB_OK;
+}
+
 extern "C" const char* pb_last_error(const pb_ctx* ctx) { return ctx ? ctx->err.c_str() : "null context"; }

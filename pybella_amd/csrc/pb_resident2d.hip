@@ -793,13 +793,11 @@ void pb2d::resident_free(pb_op2d* op) {
   op->res = nullptr;
 }
 
+namespace {
+// resident_run without its switch and counts; kGaveUp when a wait ran out
+constexpr int kGaveUp = 2;
 template <typename T>
-int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int count, bool exact, hipStream_t s,
-                       KState* out) {
-  if (ctx->resident_skip.load() > 0) {
-    ctx->resident_skip.fetch_sub(1);
-    return 0;
-  }
+int run_jobs(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int count, bool exact, hipStream_t s, KState* out) {
   for (int m = 0; m < count; ++m)   // tags of a run: three per iteration, far from wrapping
     if (jobs[m].maxiter > (1 << 28)) return 0;
   // Launches of one kind of kernel each, the members with the most tiles first,
@@ -848,6 +846,7 @@ int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int 
   ResOut* const res = (ResOut*)((char*)rec.host + tab_bytes);
   RMember<T>* const dtab = (RMember<T>*)rec.dev;
   ResOut* const dres = (ResOut*)((char*)rec.dev + tab_bytes);
+  const int give_up = ctx->resident_mode.load() == PB_RESIDENT_GIVE_UP;   // as if a wait had run out
   std::vector<int> total;
   for (int k = 0; k < count; ++k) {
     if (total.size() < spans.size() && k == spans[total.size()].f) total.push_back(0);
@@ -870,7 +869,7 @@ int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int 
     M.x0 = J.x0;
     M.x = J.x;
     M.out = dres + k;
-    res[k].abort = 0;
+    res[k].abort = give_up;
     M.halo_v = R->words;
     M.halo_t = R->words + R->halo_words;
     M.rec = R->words + 2 * R->halo_words;
@@ -898,13 +897,24 @@ int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int 
   PB_HIP(ctx, hipMemcpyAsync(res, dres, out_bytes, hipMemcpyDeviceToHost, s));
   PB_HIP(ctx, hipStreamSynchronize(s));
   for (int k = 0; k < count; ++k) {
-    if (res[k].abort) {
-      ctx->resident_skip.store(kSkipAfterAbort);
-      return 0;
-    }
+    if (res[k].abort) return kGaveUp;
   }
   for (int k = 0; k < count; ++k) out[order[k]] = res[k].st;
+  ctx->resident_count[PB_RESIDENT_LAUNCHES] += (long long)spans.size();
   return 1;
+}
+}  // namespace
+
+template <typename T>
+int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int count, bool exact, hipStream_t s,
+                       KState* out) {
+  int rc = 0;
+  if (ctx->resident_skip.load() > 0) ctx->resident_skip.fetch_sub(1);
+  else if (ctx->resident_mode.load() != PB_RESIDENT_OFF) rc = run_jobs<T>(ctx, rec, jobs, count, exact, s, out);
+  if (rc < 0) return rc;
+  ctx->resident_count[rc == 1 ? PB_RESIDENT_RUNS : rc == kGaveUp ? PB_RESIDENT_GIVEN_UP : PB_RESIDENT_DECLINED] += count;
+  if (rc == kGaveUp) ctx->resident_skip.store(kSkipAfterAbort);
+  return rc == 1;
 }
 
 template int pb2d::resident_run<double>(pb_ctx*, ResRecords&, const ResJob<double>*, int, bool, hipStream_t, KState*);

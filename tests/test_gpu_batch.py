@@ -1,7 +1,8 @@
 """GPU tests of the batched uneven solves (pb_batch_*).
 
 * FP64 (two-launch) batch: every member's solution and iteration count are
-  bitwise those of the same member solved alone with the same tile height;
+  bitwise those of the same member solved alone with the same tile height, on
+  the chip (in one launch or several) and by launches per phase;
 * mixed batch: every member reaches true relative residual 1e-8, and agrees
   with its single mixed solve to the tolerance;
 * the batched projection step equals the single drop-in per member (<= 1e-7
@@ -44,7 +45,26 @@ def _systems(members):
     return ops, bs
 
 
-def test_fp64_batch_equals_single_solves():
+@pytest.fixture(params=["resident", "launches"])
+def route(request):
+    """Both ways a batch runs; yields a check of the counts of a solve."""
+    from pybella_amd import _abi
+    ctx = _abi.default_context()
+    ctx.set_resident(_abi.PB_RESIDENT_ON if request.param == "resident" else _abi.PB_RESIDENT_OFF)
+
+    def check(solve):
+        before = ctx.resident_runs()
+        out = solve()
+        n = {k: v - before[k] for k, v in ctx.resident_runs().items()}
+        assert n["given_up"] == 0 and (n["declined"] if request.param == "resident" else n["runs"]) == 0, n
+        assert n["runs"] + n["declined"] > 0
+        return out
+
+    yield check
+    ctx.set_resident(_abi.PB_RESIDENT_ON)
+
+
+def test_fp64_batch_equals_single_solves(route):
     import torch
     from pybella_amd.batch import BatchSolver
     print("case batch f64fast", flush=True)
@@ -54,20 +74,20 @@ def test_fp64_batch_equals_single_solves():
         op.set_tile((2, 4, 8)[k % 3])          # uneven tiles across members
     singles = [op.solve(b, tol=1e-10, mode="f64fast") for op, b in zip(ops, bs)]
     singles = [(x.clone(), info) for x, info in singles]
-    xs, infos = BatchSolver(ops).solve(bs, tol=1e-10, mode="f64fast")
+    xs, infos = route(lambda: BatchSolver(ops).solve(bs, tol=1e-10, mode="f64fast"))
     torch.cuda.synchronize()
     for (xs1, i1), xb, ib in zip(singles, xs, infos):
         assert ib["info"] == 0 and ib["iters"] == i1["iters"], (ib, i1)
         assert torch.equal(xs1, xb)
 
 
-def test_mixed_batch_converges_and_agrees():
+def test_mixed_batch_converges_and_agrees(route):
     import torch
     from pybella_amd.batch import BatchSolver
     print("case batch mixed", flush=True)
     members = _members()
     ops, bs = _systems(members)
-    xs, infos = BatchSolver(ops).solve(bs, tol=1e-8, mode="mixed")
+    xs, infos = route(lambda: BatchSolver(ops).solve(bs, tol=1e-8, mode="mixed"))
     for op, b, x, info in zip(ops, bs, xs, infos):
         assert info["info"] == 0 and info["true_rel_resid"] <= 1e-8, info
         xs1, i1 = op.solve(b, tol=1e-8, mode="mixed")
@@ -118,9 +138,10 @@ def test_oracle_residual_per_member():
 
 
 @pytest.mark.parametrize("ry", [2, 5])
-def test_flattened_batch_equals_single_solves(ry):
-    """Uniform tile height: the batch runs one launch over every member's tiles
-    per phase; each member's iterates are still bitwise those of its own solve."""
+def test_flattened_batch_equals_single_solves(ry, route):
+    """Uniform tile height: the batch runs one launch over every member's tiles,
+    for the whole run or per phase; each member's iterates are still bitwise
+    those of its own solve."""
     import torch
     from pybella_amd.batch import BatchSolver
     print(f"case flattened batch ry={ry}", flush=True)
@@ -131,12 +152,35 @@ def test_flattened_batch_equals_single_solves(ry):
     singles = [op.solve(b, tol=1e-10, mode="f64fast") for op, b in zip(ops, bs)]
     singles = [(x.clone(), info) for x, info in singles]
     batch = BatchSolver(ops)
-    for _ in range(2):   # a second solve replays the captured graph
-        xs, infos = batch.solve(bs, tol=1e-10, mode="f64fast")
+    for _ in range(2):   # by launches, the second solve replays the captured graph
+        xs, infos = route(lambda: batch.solve(bs, tol=1e-10, mode="f64fast"))
         torch.cuda.synchronize()
         for (xs1, i1), xb, ib in zip(singles, xs, infos):
             assert ib["info"] == 0 and ib["iters"] == i1["iters"], (ib, i1)
             assert torch.equal(xs1, xb)
-    xs, infos = batch.solve(bs, tol=1e-8, mode="mixed")
+    xs, infos = route(lambda: batch.solve(bs, tol=1e-8, mode="mixed"))
     for op, b, info in zip(ops, bs, infos):
         assert info["info"] == 0 and info["true_rel_resid"] <= 1e-8, info
+
+
+def test_batch_of_more_tiles_than_are_resident_at_once():
+    """Twelve members of 85 tiles and four smaller ones, one group: their 1046
+    tiles go in two launches, each member's result bitwise that of its own
+    solve by launches per phase."""
+    import torch
+    from pybella_amd.batch import BatchSolver
+    print("case batch in several launches", flush=True)
+    members = [W.batch_member_bubble(257, 129, m) for m in range(12)]
+    members[3:3] = [W.batch_member_bubble(nx, ny, 1) for nx, ny in SIZES[:2] * 2]
+    ops, bs = _systems(members)
+    for op in ops:
+        op.set_tile(2)
+    singles = [op.solve_noalloc(b, torch.full_like(b, np.nan), tol=1e-10, mode="f64fast") for op, b in zip(ops, bs)]
+    batch, ctx = BatchSolver(ops), ops[0].ctx
+    for _ in range(2):
+        before = ctx.resident_runs()
+        xs, infos = batch.solve(bs, tol=1e-10, mode="f64fast")
+        n = {k: v - before[k] for k, v in ctx.resident_runs().items()}
+        assert n == dict(runs=16, launches=2, declined=0, given_up=0), n
+        for (x1, i1), x, i in zip(singles, xs, infos):
+            assert i["info"] == 0 and i["iters"] == i1["iters"] and torch.equal(x1, x), (i, i1)

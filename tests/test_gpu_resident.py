@@ -2,7 +2,8 @@
 launch-per-phase iteration: same tiles, same operations, same summation
 orders, so x, the iteration count and the info are bitwise equal.
 
-``solve_noalloc`` always runs the launches.  The grids cover a single tile,
+``solve_noalloc`` always runs the launches, and the context's counts say that
+``solve`` did not.  The grids cover a single tile,
 tiles cut at the last row and column, wraps inside one tile, each way of
 summing the records (one wave, several waves, class sums), more tiles than
 two per compute unit, and a grid too large to be resident."""
@@ -28,9 +29,20 @@ def _system(nx, ny, kind, seed=17):
     return op, op.scale_rhs(sp.to_dev(W.stratified_rhs(node, seed=seed)))
 
 
+def _counted(op, solve):
+    """solve(), and what it added to the context's counts of resident runs."""
+    before = op.ctx.resident_runs()
+    out = solve()
+    return out, {k: n - before[k] for k, n in op.ctx.resident_runs().items()}
+
+
+ONE = dict(runs=1, launches=1, declined=0, given_up=0)
+
+
 def _same(op, b, **kw):
     import torch
-    x1, i1 = op.solve(b, **kw)
+    (x1, i1), n = _counted(op, lambda: op.solve(b, **kw))
+    assert n == ONE, n
     x2, i2 = op.solve_noalloc(b, torch.full_like(b, np.nan), **kw)
     torch.cuda.synchronize()
     assert i1["iters"] == i2["iters"] and i1["info"] == i2["info"] and i1["half_step"] == i2["half_step"], (i1, i2)
@@ -78,7 +90,8 @@ def test_more_tiles_than_two_per_unit_and_guess():
     print("case resident 1025x513 ry 4, guess, zero rhs", flush=True)
     op, b = _system(1025, 513, "coriolis")
     x, _ = _same(op, b, tol=1e-30, maxiter=40, mode="f64fast")
-    x1, i1 = op.solve(b, tol=1e-8, maxiter=6000, mode="f64", x0=x)
+    (x1, i1), n = _counted(op, lambda: op.solve(b, tol=1e-8, maxiter=6000, mode="f64", x0=x))
+    assert n == ONE, n
     x2, i2 = op.solve_noalloc(b, x.clone(), tol=1e-8, maxiter=6000, mode="f64", x0_given=True)
     assert i1["iters"] == i2["iters"] and torch.equal(x1, x2) and i1["info"] == 0
     z, iz = op.solve(torch.zeros_like(b), tol=1e-8, mode="f64fast")
@@ -87,7 +100,7 @@ def test_more_tiles_than_two_per_unit_and_guess():
 
 
 def test_too_large_to_be_resident_and_two_streams():
-    """1025 x 1025 with 8-row tiles (more than 768) runs by launches; solves
+    """1025 x 1025 with 2-row threads (8-row tiles, more than 768) runs by launches; solves
     from two threads, on their own contexts and streams and on the default
     one with an operator each, share the device's room."""
     import threading
@@ -98,7 +111,8 @@ def test_too_large_to_be_resident_and_two_streams():
     print("case resident 1025x1025 ry 2, two threads", flush=True)
     op, b = _system(1025, 1025, "comp")
     op.set_tile(2)
-    x, info = op.solve(b, tol=1e-8, mode="f64fast")
+    (x, info), n = _counted(op, lambda: op.solve(b, tol=1e-8, mode="f64fast"))
+    assert n == dict(runs=0, launches=0, declined=1, given_up=0), n
     assert info["info"] == 0 and info["true_rel_resid"] < 2e-8
     op.close()
     op, b = _system(257, 129, "psinc")
@@ -130,4 +144,37 @@ def test_too_large_to_be_resident_and_two_streams():
             t.join()
     assert not err, err
     assert all(torch.equal(g, ref) for g in got)
+    op.close()
+
+
+@pytest.mark.parametrize("nx,ny,mode", [(61, 15, "f64"), (161, 81, "f64fast"), (161, 81, "mixed"), (301, 301, "f64"),
+                                        (513, 257, "f64fast")])
+def test_given_up_runs_are_repeated_by_launches(nx, ny, mode):
+    """Every run given up by its abort word, set beforehand: blocks leave at
+    their next wait (or end, x written), and the launches repeat the run.  Same
+    solution as without, with and without a guess; the next solves go by
+    launches at once, until the switch is set again."""
+    import torch
+    from pybella_amd import _abi
+    print(f"case given up {nx}x{ny} {mode}", flush=True)
+    op, b = _system(nx, ny, "coriolis")
+    guess = torch.from_numpy(np.random.default_rng(3).standard_normal((ny, nx))).cuda()
+    kws = [dict(tol=1e-8, mode=mode)] + ([dict(tol=1e-8, mode=mode, x0=guess)] if mode != "mixed" else [])
+    ctx = op.ctx
+    try:
+        for kw in kws:
+            ctx.set_resident(_abi.PB_RESIDENT_OFF)
+            (x1, i1), n = _counted(op, lambda: op.solve(b, **kw))
+            assert n["runs"] == n["given_up"] == 0 and n["declined"] >= 1, n
+            ctx.set_resident(_abi.PB_RESIDENT_GIVE_UP)
+            (x2, i2), n = _counted(op, lambda: op.solve(b, **kw))
+            assert n["runs"] == 0 and n["given_up"] == 1, n
+            assert i1["info"] == i2["info"] == 0 and i1["iters"] == i2["iters"] and torch.equal(x1, x2)
+            (x2, i2), n = _counted(op, lambda: op.solve(b, **kw))
+            assert n["runs"] == n["given_up"] == 0 and n["declined"] >= 1 and torch.equal(x1, x2), n
+            ctx.set_resident(_abi.PB_RESIDENT_ON)
+            (x2, i2), n = _counted(op, lambda: op.solve(b, **kw))
+            assert n["runs"] >= 1 and n["declined"] == 0 and torch.equal(x1, x2), n
+    finally:
+        ctx.set_resident(_abi.PB_RESIDENT_ON)
     op.close()
