@@ -158,11 +158,16 @@ int pb_ctx_destroy(pb_ctx* ctx);
 int pb_ctx_set_stream(pb_ctx* ctx, void* hip_stream);
 int pb_ctx_synchronize(pb_ctx* ctx);
 /* Whether the context's BiCGStab runs may stay on the chip (one launch per run,
- * PB_RESIDENT_ON at first); results are the same bit for bit.  Also ends the
- * pause after runs that were given up. */
+ * PB_RESIDENT_ON at first); results are the same bit for bit.  After a run that
+ * was given up (its blocks were not all on the device at once, as beside another
+ * process) the next 64 go by launches, after three all do, until this is called
+ * again. */
 int pb_ctx_set_resident(pb_ctx* ctx, int mode);
 /* counts[PB_RESIDENT_COUNTS] since the context was made */
 int pb_ctx_resident_runs(const pb_ctx* ctx, int64_t* counts);
+/* Compute units of n_cu that a run of ``tiles`` tiles is charged while it is on
+ * the chip; runs are admitted while their charges fit.  Host only. */
+int pb_resident_units(int tiles, int n_cu);
 const char* pb_last_error(const pb_ctx* ctx);
 
 /* cell ghost fill: wrap / mirror in x, hydrostatic images in y (gravity axis).

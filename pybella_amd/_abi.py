@@ -87,6 +87,7 @@ SIGNATURES = {
     "pb_ctx_synchronize": (I, [VP]),
     "pb_ctx_set_resident": (I, [VP, I]),
     "pb_ctx_resident_runs": (I, [VP, C.c_int64 * 4]),
+    "pb_resident_units": (I, [I, I]),
     "pb_last_error": (C.c_char_p, [VP]),
     "pb_bc_cells": (I, [VP, C.POINTER(Grid2D), C.POINTER(Phys), VP * 6, VP]),
     "pb_ghostnodes": (I, [VP, C.POINTER(Grid2D), VP]),

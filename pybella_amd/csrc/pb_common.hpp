@@ -20,9 +20,10 @@ struct pb_ctx {
   double* scratch = nullptr;
   size_t scratch_bytes = 0;
   int scratch_err = 0;   // hipError_t of the address lookup
-  // resident Krylov runs: PB_RESIDENT_*, runs still to do by launches after a
-  // wait ran out, and the counts that pb_ctx_resident_runs gives
+  // resident Krylov runs: PB_RESIDENT_*, how often a wait ran out, runs still to
+  // do by launches since, and the counts that pb_ctx_resident_runs gives
   std::atomic<int> resident_mode{PB_RESIDENT_ON};
+  std::atomic<int> resident_give_ups{0};
   std::atomic<int> resident_skip{0};
   std::atomic<long long> resident_count[PB_RESIDENT_COUNTS] = {};
 };

@@ -95,6 +95,7 @@ extern "C" int pb_ctx_set_resident(pb_ctx* ctx, int mode) {
     return pb_fail(ctx, PB_ERR_ARG, "pb_ctx_set_resident: mode %d", mode);
   ctx->resident_mode.store(mode);
   ctx->resident_skip.store(0);
+  ctx->resident_give_ups.store(0);
   return PB_OK;
 }
 

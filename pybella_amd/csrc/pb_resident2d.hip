@@ -39,8 +39,10 @@
 //
 // Every wait is bounded (kWaitTicks).  When one runs out, because the blocks
 // are not all resident next to other work, the launch ends without a result
-// and the caller runs the launches; room is accounted for per device so that
-// runs of several streams or threads are not resident in part.
+// and the caller runs the launches.  Room is accounted for per device, so that
+// runs of several streams or threads of a process are not resident in part; for
+// what the account does not see, as another process on the device, the wait is
+// short and a context that has given up kMaxGiveUps times stops trying.
 #include <atomic>
 #include <type_traits>
 #include <vector>
@@ -87,8 +89,9 @@ constexpr int kDirect = 96;          // tiles up to which every block sums the r
 constexpr int kMaxPerLane = 3;       // records of a class sum's lane: up to 768 tiles
 constexpr int kCopies = 8;           // copies of the class sums
 constexpr int kSumWords = 64;        // words of one copy's class sums (<= 40 used)
-constexpr long long kWaitTicks = 200000000LL;   // 2 s of the 100 MHz clock
+constexpr long long kWaitTicks = 20000000LL;   // 0.2 s of the 100 MHz clock; a phase takes ~10 us
 constexpr int kSkipAfterAbort = 64;  // solves of a context that go by launches after a wait ran out
+constexpr int kMaxGiveUps = 3;       // and after so many, all of them
 
 template <typename T>
 struct RMember {
@@ -683,9 +686,16 @@ __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __res
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// Compute units taken by resident launches, per device: a launch starts only
-// when its blocks fit beside those already running, so no two of them wait
-// for room that the other holds.
+// Compute units (CUs) taken by resident launches, per device.  A launch of at
+// most a block per CU is charged a CU per block, rounded up to the same number on
+// every XCD: blocks go to the XCDs in turn and spread over their CUs, and a CU
+// that holds blocks of one kind may have no registers or LDS left for another.
+// So on every XCD each run finds as many CUs without foreign blocks as it has
+// blocks there.  A larger launch, several blocks to a CU, is charged the device
+// and runs alone; a run that finds no room goes by launches.
+constexpr int kXcds = 8;
+int units_of(int tiles, int n_cu) { return std::min(n_cu, ceil_div(tiles, kXcds) * kXcds); }
+
 constexpr int kMaxDev = 64;
 std::atomic<int> g_cus_taken[kMaxDev];
 
@@ -833,7 +843,7 @@ int run_jobs(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int count, boo
     if (tiles(order[f]) > std::min(slots, kMaxPerLane * NTHR)) return 0;
     int e = f, total = 0;
     while (e < count && kind(order[e]) == kind(order[f]) && total + tiles(order[e]) <= slots) total += tiles(order[e++]);
-    need = std::max(need, std::min(ctx->n_cu, ceil_div(total, occ)));
+    need = std::max(need, units_of(total, ctx->n_cu));
     spans.push_back(Span{f, e, fn});
     f = e;
   }
@@ -909,13 +919,19 @@ template <typename T>
 int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int count, bool exact, hipStream_t s,
                        KState* out) {
   int rc = 0;
-  if (ctx->resident_skip.load() > 0) ctx->resident_skip.fetch_sub(1);
-  else if (ctx->resident_mode.load() != PB_RESIDENT_OFF) rc = run_jobs<T>(ctx, rec, jobs, count, exact, s, out);
+  const bool on = ctx->resident_mode.load() != PB_RESIDENT_OFF && ctx->resident_give_ups.load() < kMaxGiveUps;
+  if (on && ctx->resident_skip.load() > 0) ctx->resident_skip.fetch_sub(1);
+  else if (on) rc = run_jobs<T>(ctx, rec, jobs, count, exact, s, out);
   if (rc < 0) return rc;
   ctx->resident_count[rc == 1 ? PB_RESIDENT_RUNS : rc == kGaveUp ? PB_RESIDENT_GIVEN_UP : PB_RESIDENT_DECLINED] += count;
-  if (rc == kGaveUp) ctx->resident_skip.store(kSkipAfterAbort);
+  if (rc == kGaveUp) {
+    ctx->resident_give_ups.fetch_add(1);
+    ctx->resident_skip.store(kSkipAfterAbort);
+  }
   return rc == 1;
 }
+
+extern "C" int pb_resident_units(int tiles, int n_cu) { return tiles < 1 || n_cu < 1 ? PB_ERR_ARG : units_of(tiles, n_cu); }
 
 template int pb2d::resident_run<double>(pb_ctx*, ResRecords&, const ResJob<double>*, int, bool, hipStream_t, KState*);
 template int pb2d::resident_run<float>(pb_ctx*, ResRecords&, const ResJob<float>*, int, bool, hipStream_t, KState*);

@@ -178,3 +178,25 @@ def test_given_up_runs_are_repeated_by_launches(nx, ny, mode):
     finally:
         ctx.set_resident(_abi.PB_RESIDENT_ON)
     op.close()
+
+
+def test_a_context_stops_trying_after_three_given_up_runs():
+    """64 solves by launches after each given-up run, all after the third."""
+    from pybella_amd import _abi
+    print("case resident given up three times", flush=True)
+    op, b = _system(33, 17, "psinc")
+    ctx = op.ctx
+    ref, _ = op.solve(b, mode="f64fast")
+    try:
+        ctx.set_resident(_abi.PB_RESIDENT_GIVE_UP)
+        gave_up = []
+        for k in range(3 * 65 + 70):
+            _, n = _counted(op, lambda: op.solve(b, mode="f64fast"))
+            assert n["runs"] == 0 and n["given_up"] + n["declined"] == 1
+            gave_up += [k] * n["given_up"]
+        assert gave_up == [0, 65, 130], gave_up
+    finally:
+        ctx.set_resident(_abi.PB_RESIDENT_ON)
+    (x, _), n = _counted(op, lambda: op.solve(b, mode="f64fast"))
+    assert n == ONE and bool((x == ref).all())
+    op.close()
