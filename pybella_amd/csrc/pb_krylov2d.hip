@@ -1255,11 +1255,10 @@ int krylov_run(pb_op2d* op, Work<T>& w, const T* b, const double* x0, double tol
   if (!host && !fused) {
     // a grid whose tiles are all resident iterates in one launch; the init
     // launch forms b - A x0 when a guess is given
-    if (x0) launch_init();
     const ResJob<T> job{op, b, x0 ? w.r[0] : b, x0 ? w.x : nullptr, w.x, tol, maxiter, legacy};
-    Resident* R = resident_of(op);
-    if (!R) return PB_ERR_HIP;
-    const int rc = resident_run<T>(ctx, R->records, &job, 1, exact, s, out);
+    const int rc = resident_run<T>(ctx, resident_of(op)->records, &job, 1, exact, s, out, [&] {
+      if (x0) launch_init();
+    });
     if (rc != 0) return rc < 0 ? rc : PB_OK;
   }
   KState init{};

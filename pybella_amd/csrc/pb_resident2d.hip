@@ -755,24 +755,42 @@ ResKernel<T> pick(int ry, bool cross, bool center, bool exact, bool many) {
 
 constexpr long kSumsAll = (long)kRecValues * kCopies * kSumWords;
 
-int ensure_records(pb_ctx* ctx, ResRecords& rec, size_t bytes, hipStream_t s) {
+// Memory of the resident runs, taken once a run is known to fit.  Without it the
+// runs go by launches, which need none of it: false, and no error left behind.
+bool take(hipError_t e) {
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e == hipSuccess;
+}
+
+bool ensure_records(ResRecords& rec, size_t bytes, hipStream_t s) {
   if (!rec.ticket) {
     void* p = nullptr;
-    PB_HIP(ctx, hipMalloc(&p, 256));
+    if (!take(hipMalloc(&p, 256))) return false;
     rec.ticket = (unsigned*)p;
     rec.ticket_next = 0;
     hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(64), 0, s, 32L, (u64*)p);
-    PB_LAUNCH_CHECK(ctx);
   }
-  if (rec.bytes >= bytes) return PB_OK;
+  if (rec.bytes >= bytes) return true;
   if (rec.dev) (void)hipFree(rec.dev);
   if (rec.host) (void)hipHostFree(rec.host);
   rec.dev = rec.host = nullptr;
   rec.bytes = 0;
-  PB_HIP(ctx, hipMalloc(&rec.dev, bytes));
-  PB_HIP(ctx, hipHostMalloc(&rec.host, bytes, hipHostMallocDefault));
+  if (!take(hipMalloc(&rec.dev, bytes)) || !take(hipHostMalloc(&rec.host, bytes, hipHostMallocDefault))) return false;
   rec.bytes = bytes;
-  return PB_OK;
+  return true;
+}
+
+bool ensure_words(pb_op2d* op) {
+  Resident* R = resident_of(op);
+  if (R->words) return true;
+  // sized for the finest tiling, so every tile height uses the same buffers
+  const dim3 g = stencil_grid(op, 2);
+  R->halo_words = 2 * ((2L * g.y + 2) * op->g.nx + (2L * g.x + 2) * op->g.ny);
+  R->rec_words = 2L * kRecValues * g.x * g.y;
+  void* p = nullptr;
+  if (!take(hipMalloc(&p, sizeof(u64) * (2 * R->halo_words + R->rec_words + kSumsAll)))) return false;
+  R->words = (u64*)p;
+  return true;
 }
 
 }  // namespace
@@ -785,21 +803,15 @@ void pb2d::ResRecords::release() {
 }
 
 Resident* pb2d::resident_of(pb_op2d* op) {
-  if (op->res) return op->res;
-  // sized for the finest tiling, so every tile height uses the same buffers
-  const dim3 g = stencil_grid(op, 2);
-  Resident R;
-  R.halo_words = 2 * ((2L * g.y + 2) * op->g.nx + (2L * g.x + 2) * op->g.ny);
-  R.rec_words = 2L * kRecValues * g.x * g.y;
-  if (dmalloc(op, &R.words, 2 * R.halo_words + R.rec_words + kSumsAll)) return nullptr;
-  op->res = new Resident(R);
+  if (!op->res) op->res = new Resident();
   return op->res;
 }
 
 void pb2d::resident_free(pb_op2d* op) {
   if (!op->res) return;
   op->res->records.release();
-  delete op->res;   // its device words are in op->allocs
+  if (op->res->words) (void)hipFree(op->res->words);
+  delete op->res;
   op->res = nullptr;
 }
 
@@ -807,7 +819,8 @@ namespace {
 // resident_run without its switch and counts; kGaveUp when a wait ran out
 constexpr int kGaveUp = 2;
 template <typename T>
-int run_jobs(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int count, bool exact, hipStream_t s, KState* out) {
+int run_jobs(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int count, bool exact, hipStream_t s, KState* out,
+             const std::function<void()>& prepare) {
   for (int m = 0; m < count; ++m)   // tags of a run: three per iteration, far from wrapping
     if (jobs[m].maxiter > (1 << 28)) return 0;
   // Launches of one kind of kernel each, the members with the most tiles first,
@@ -850,8 +863,10 @@ int run_jobs(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int count, boo
   Room room;
   if (!room.acquire(ctx->device, need, ctx->n_cu)) return 0;
   const size_t tab_bytes = (sizeof(RMember<T>) * count + 255) / 256 * 256, out_bytes = sizeof(ResOut) * count;
-  int rc = ensure_records(ctx, rec, tab_bytes + out_bytes, s);
-  if (rc) return rc;
+  if (!ensure_records(rec, tab_bytes + out_bytes, s)) return 0;
+  for (int m = 0; m < count; ++m)
+    if (!ensure_words(jobs[m].op)) return 0;
+  if (prepare) prepare();
   RMember<T>* const tab = (RMember<T>*)rec.host;
   ResOut* const res = (ResOut*)((char*)rec.host + tab_bytes);
   RMember<T>* const dtab = (RMember<T>*)rec.dev;
@@ -862,8 +877,7 @@ int run_jobs(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int count, boo
     if (total.size() < spans.size() && k == spans[total.size()].f) total.push_back(0);
     const ResJob<T>& J = jobs[order[k]];
     pb_op2d* op = J.op;
-    Resident* R = resident_of(op);
-    if (!R) return PB_ERR_HIP;
+    Resident* R = op->res;
     const u32 span = 3u * (u32)J.maxiter + 8u;
     if (!R->cleared || R->epoch > 0xffffffffu - span) {
       const long words = 2 * R->halo_words + R->rec_words + kSumsAll;
@@ -917,11 +931,11 @@ int run_jobs(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int count, boo
 
 template <typename T>
 int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int count, bool exact, hipStream_t s,
-                       KState* out) {
+                       KState* out, const std::function<void()>& prepare) {
   int rc = 0;
   const bool on = ctx->resident_mode.load() != PB_RESIDENT_OFF && ctx->resident_give_ups.load() < kMaxGiveUps;
   if (on && ctx->resident_skip.load() > 0) ctx->resident_skip.fetch_sub(1);
-  else if (on) rc = run_jobs<T>(ctx, rec, jobs, count, exact, s, out);
+  else if (on) rc = run_jobs<T>(ctx, rec, jobs, count, exact, s, out, prepare);
   if (rc < 0) return rc;
   ctx->resident_count[rc == 1 ? PB_RESIDENT_RUNS : rc == kGaveUp ? PB_RESIDENT_GIVEN_UP : PB_RESIDENT_DECLINED] += count;
   if (rc == kGaveUp) {
@@ -933,5 +947,7 @@ int pb2d::resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int 
 
 extern "C" int pb_resident_units(int tiles, int n_cu) { return tiles < 1 || n_cu < 1 ? PB_ERR_ARG : units_of(tiles, n_cu); }
 
-template int pb2d::resident_run<double>(pb_ctx*, ResRecords&, const ResJob<double>*, int, bool, hipStream_t, KState*);
-template int pb2d::resident_run<float>(pb_ctx*, ResRecords&, const ResJob<float>*, int, bool, hipStream_t, KState*);
+template int pb2d::resident_run<double>(pb_ctx*, ResRecords&, const ResJob<double>*, int, bool, hipStream_t, KState*,
+                                        const std::function<void()>&);
+template int pb2d::resident_run<float>(pb_ctx*, ResRecords&, const ResJob<float>*, int, bool, hipStream_t, KState*,
+                                       const std::function<void()>&);

@@ -1,6 +1,8 @@
 // Host interface of the resident BiCGStab (pb_resident2d.hip): whole Krylov
 // runs in one launch, the vectors held in registers.
 #pragma once
+#include <functional>
+
 #include "pb_bicg2d.hpp"
 
 namespace pb2d {
@@ -26,7 +28,7 @@ struct ResRecords {
 
 // Device words of one operator's resident runs: the edge exchange, the
 // partial records and their sums, all tagged.  One allocation, made at the
-// first run.
+// first run that fits on the chip.
 struct Resident {
   unsigned long long* words = nullptr;
   long halo_words = 0;   // of one exchange buffer (there are two)
@@ -47,18 +49,19 @@ struct ResJob {
   int maxiter, legacy;
 };
 
-// The operator's Resident, made at the first call; null (and an error on the
-// context) when its memory cannot be had.
+// The operator's Resident, made at the first call, still without device memory.
 Resident* resident_of(pb_op2d* op);
 
-// Run every job in one launch per operator kind, with the launch records
-// ``rec`` of their owner.  Returns 1 with the final
-// states in ``out`` when all of them ran, 0 when the launch does not apply
-// here (grid too large to be resident, no free room, or a wait ran out: the
-// caller takes the launch-per-phase path), < 0 on an error.
+// Run every job with the launch records ``rec`` of their owner, in as few
+// launches as the operator kinds and the tiles resident at once allow.
+// ``prepare`` issues on ``s`` what the jobs' inputs still need; it is called once
+// the runs are known to fit.  Returns 1 with the final states in ``out`` when all
+// of them ran, 0 when they do not apply here (grid too large to be resident, no
+// free room or memory, or a wait ran out: the caller takes the launch-per-phase
+// path), < 0 on an error.
 template <typename T>
 int resident_run(pb_ctx* ctx, ResRecords& rec, const ResJob<T>* jobs, int count, bool exact, hipStream_t s,
-                 KState* out);
+                 KState* out, const std::function<void()>& prepare = {});
 
 void resident_free(pb_op2d* op);
 

@@ -200,3 +200,21 @@ def test_a_context_stops_trying_after_three_given_up_runs():
     (x, _), n = _counted(op, lambda: op.solve(b, mode="f64fast"))
     assert n == ONE and bool((x == ref).all())
     op.close()
+
+
+def test_a_grid_too_large_takes_no_memory_for_it():
+    """2049 x 1025 nodes (2145 tiles) can never be resident: its solve, with a
+    guess too, takes none of the exchange words (19 MB at this size)."""
+    import torch
+    print("case resident 2049x1025 memory", flush=True)
+    op, b = _system(2049, 1025, "psinc")
+    op.time_kernel(0, reps=1)   # the solver's vectors
+    x, guess = torch.empty_like(b), torch.zeros_like(b)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    for kw in (dict(mode="f64fast"), dict(mode="f64", x0=guess)):
+        _, n = _counted(op, lambda: op.solve(b, x=x, tol=1e-30, maxiter=1, **kw))
+        assert n["declined"] == 1 and n["runs"] == 0
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < 12 << 20
+    op.close()
