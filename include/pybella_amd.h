@@ -422,8 +422,8 @@ int pb_op2d_mg_features(pb_op2d* op, float* f1, float* f2);
  * (src/__main__.py:223-254, each through second_projection.py:230).  A batch
  * holds distinct assembled operators (one per member, each with its own tile
  * height); members run as resident launches where their tiles fit on the
- * chip, else as chunks of iterations of every member in one hipGraph, replayed
- * until all members are final.  Per member the iterates equal a single
+ * chip, else the members of one kind (tile height, cross and centre terms) share
+ * a hipGraph per chunk of iterations, replayed until they are final.  Per member the iterates equal a single
  * solve's. */
 int pb_batch_create(pb_ctx* ctx, pb_op2d* const* ops, int count, pb_batch** out);
 int pb_batch_destroy(pb_batch* batch);

@@ -1,7 +1,8 @@
 """Batched uneven 2D solves (pb_batch_*): many assembled operators, possibly
 of different grid sizes, solved together: resident launches for members whose
-tiles fit on the chip, else one hipGraph per chunk of iterations.  No reference counterpart: the reference
-solves ensemble members one after the other (src/__main__.py:223-254)."""
+tiles fit on the chip, else one hipGraph per chunk of iterations and kind of
+member.  No reference counterpart: the reference solves ensemble members one
+after the other (src/__main__.py:223-254)."""
 from __future__ import annotations
 
 import ctypes as C

@@ -1811,13 +1811,14 @@ extern "C" int pb_op2d_set_tile(pb_op2d* op, int rows_per_thread) {
 // ---------------------------------------------------------------------------
 // Batched uneven solves (ensemble members, possibly of different grid sizes).
 // Every member keeps its own operator, workspace, tile height and kernels, so
-// its iterates are those of a single solve.  A chunk of iterations of ALL
-// members is captured as one hipGraph: a fork from the caller's stream into
-// one branch per member stream, joined back at the end.  Each replay advances
-// every member by the chunk; members that have finished run no-op launches
-// (their state is final).  The host reads all members' states once per chunk.
-// No reference counterpart: the reference solves ensemble members one after
-// the other (src/__main__.py:223-254).
+// its iterates are those of a single solve.  Where the members' tiles fit on the
+// chip they run as resident launches (pb_resident2d.hip).  Else the members of
+// one kind (tile height, cross and centre terms) share flattened launches, one
+// grid over the tiles of all of them per phase, captured as one hipGraph per
+// chunk of iterations; the kinds run in turn.  Members that have finished run
+// no-op launches (their state is final).  The host reads all members' states
+// once per chunk.  No reference counterpart: the reference solves ensemble
+// members one after the other (src/__main__.py:223-254).
 // ---------------------------------------------------------------------------
 struct pb_batch {
   pb_ctx* ctx = nullptr;
@@ -1825,13 +1826,8 @@ struct pb_batch {
   void* mtab[2] = {nullptr, nullptr};      // device member tables (FP64, FP32) of the flattened launches
   KState* dstates = nullptr;               // device gather target, one per member
   std::vector<char> htab[2];               // host images of the member tables
-  std::map<long, hipGraphExec_t> flat_graphs;
-  int flat_sig = -1;                       // (ry, cross, center) the flat graphs were captured with
-  std::vector<hipStream_t> streams;
-  hipEvent_t fork = nullptr;
-  std::vector<hipEvent_t> joins;
-  std::map<long, hipGraphExec_t> graphs;   // key: precision, chunk
-  std::vector<int> ry_captured;            // member launch signatures the graphs were captured with
+  std::map<std::pair<int, long>, hipGraphExec_t> graphs;   // key: kind; chunk and precision
+  std::vector<int> kinds;                  // the members' kinds the graphs were captured with
   KState* hst = nullptr;                   // pinned, one per member
   pb2d::ResRecords records;                // of the resident runs
   // a user-facing batch is split into groups (each a batch of its own) whose
@@ -1961,40 +1957,30 @@ __global__ void k_gather_states(const BMember<T>* mem, int nmem, int slot, KStat
 #define PB_FLAT(KERNEL, T, cross, center, ry, grd, s, ...) \
   PB_RY_SWITCH(ry, PB_FLAT_AT, KERNEL, T, cross, center, grd, s, __VA_ARGS__)
 
-// the batch can use the flattened launches when every member has the same
-// tile height and operator kind; returns the (ry, cross, center) signature or -1
-int flat_signature(const pb_batch* bt) {
-  const pb_op2d* o0 = bt->ops[0];
-  for (const pb_op2d* op : bt->ops)
-    if (op->ry != o0->ry || op->cross != o0->cross || op->center != o0->center) return -1;
-  return o0->ry * 4 + (o0->cross ? 2 : 0) + (o0->center ? 1 : 0);
-}
+// launch signature of a member: tile height and (cross, center)
+int kind_of(const pb_op2d* op) { return op->ry * 4 + (op->cross ? 2 : 0) + (op->center ? 1 : 0); }
 
+// One Krylov run of the members ``who``, all of one kind: member m's state goes
+// to out[m].
 template <typename T>
-int krylov_batch_flat(pb_batch* bt, const std::vector<char>& active, const std::vector<const T*>& b,
-                      const std::vector<double>& tol, int maxiter, int legacy, int check_every, hipStream_t s,
-                      std::vector<KState>& out) {
+int krylov_batch_flat(pb_batch* bt, const std::vector<int>& who, const std::vector<char>& active,
+                      const std::vector<const T*>& b, const std::vector<double>& tol, int maxiter, int legacy,
+                      int check_every, hipStream_t s, std::vector<KState>& out) {
   const int P = std::is_same<T, float>::value ? 1 : 0;
-  const int M = (int)bt->ops.size();
-  const pb_op2d* o0 = bt->ops[0];
+  const int M = (int)who.size();
+  const pb_op2d* o0 = bt->ops[who[0]];
   const int ry = o0->ry;
   const bool cross = o0->cross, center = o0->center;
-  const int sig = flat_signature(bt);
-  if (sig != bt->flat_sig) {   // captured launches are specialised on the signature
-    for (auto& kv : bt->flat_graphs) (void)hipGraphExecDestroy(kv.second);
-    bt->flat_graphs.clear();
-    bt->flat_sig = sig;
-  }
   // member table (device pointers are fixed for the life of the workspaces)
   std::vector<BMember<T>> tab((size_t)M);
   int total = 0;
   for (int m = 0; m < M; ++m) {
-    pb_op2d* op = bt->ops[m];
+    pb_op2d* op = bt->ops[who[m]];
     Work<T>& w = work_of<T>(op);
     const dim3 g = stencil_grid(op, ry);
     BMember<T>& e = tab[(size_t)m];
     e.op = opdev<T>(op);
-    e.b = b[m];
+    e.b = b[who[m]];
     for (int q = 0; q < 2; ++q) {
       e.r[q] = w.r[q];
       e.p[q] = w.p[q];
@@ -2017,15 +2003,15 @@ int krylov_batch_flat(pb_batch* bt, const std::vector<char>& active, const std::
   PB_HIP(bt->ctx, hipMemcpyAsync(bt->mtab[P], ht.data(), ht.size(), hipMemcpyHostToDevice, s));
   for (int m = 0; m < M; ++m) {
     KState init{};
-    init.tol = tol[(size_t)m];
+    init.tol = tol[who[m]];
     init.maxiter = maxiter;
     init.legacy = legacy;
     init.phase = PH_INIT;
-    init.status = active[(size_t)m] ? ST_RUN : ST_CONV;
+    init.status = active[who[m]] ? ST_RUN : ST_CONV;
     bt->hst[m] = init;
-    Work<T>& w = work_of<T>(bt->ops[m]);
+    Work<T>& w = work_of<T>(bt->ops[who[m]]);
     PB_HIP(bt->ctx, hipMemcpyAsync(w.S, bt->hst + m, sizeof(KState), hipMemcpyHostToDevice, s));
-    if (!active[(size_t)m])
+    if (!active[who[m]])
       PB_HIP(bt->ctx, hipMemcpyAsync(w.S + 1, bt->hst + m, sizeof(KState), hipMemcpyHostToDevice, s));
   }
   const BMember<T>* dt = (const BMember<T>*)bt->mtab[P];
@@ -2044,16 +2030,16 @@ int krylov_batch_flat(pb_batch* bt, const std::vector<char>& active, const std::
   };
   hipGraphExec_t ex = nullptr;
   if (graphs) {
-    const long key = ((long)chunk * 2 + P) * 65536 + total;
-    auto it = bt->flat_graphs.find(key);
-    if (it == bt->flat_graphs.end()) {
+    const std::pair<int, long> key(kind_of(o0), (long)chunk * 2 + P);
+    auto it = bt->graphs.find(key);
+    if (it == bt->graphs.end()) {
       hipGraph_t gr = nullptr;
       PB_HIP(bt->ctx, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
       issue_chunk();
       PB_HIP(bt->ctx, hipStreamEndCapture(s, &gr));
       PB_HIP(bt->ctx, hipGraphInstantiate(&ex, gr, nullptr, nullptr, 0));
       (void)hipGraphDestroy(gr);
-      it = bt->flat_graphs.emplace(key, ex).first;
+      it = bt->graphs.emplace(key, ex).first;
     }
     ex = it->second;
   }
@@ -2072,38 +2058,7 @@ int krylov_batch_flat(pb_batch* bt, const std::vector<char>& active, const std::
     PB_LAUNCH_CHECK(bt->ctx);
     issued += chunk;
   }
-  out.assign(bt->hst, bt->hst + M);
-  return PB_OK;
-}
-
-template <typename T>
-int batch_graph(pb_batch* bt, int chunk, hipStream_t s, hipGraphExec_t* out) {
-  std::vector<int> ry;   // launch signature of every member: tile height and (cross, center)
-  for (pb_op2d* op : bt->ops) ry.push_back(op->ry * 4 + (op->cross ? 2 : 0) + (op->center ? 1 : 0));
-  if (ry != bt->ry_captured) {   // a member's tile or operator kind changed: the launches are stale
-    for (auto& kv : bt->graphs) (void)hipGraphExecDestroy(kv.second);
-    bt->graphs.clear();
-    bt->ry_captured = ry;
-  }
-  const long key = (long)chunk * 2 + (std::is_same<T, float>::value ? 1 : 0);
-  auto it = bt->graphs.find(key);
-  if (it == bt->graphs.end()) {
-    hipGraph_t gr = nullptr;
-    hipGraphExec_t ex = nullptr;
-    PB_HIP(bt->ctx, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    PB_HIP(bt->ctx, hipEventRecord(bt->fork, s));
-    for (size_t m = 0; m < bt->ops.size(); ++m) {
-      PB_HIP(bt->ctx, hipStreamWaitEvent(bt->streams[m], bt->fork, 0));
-      launch_chunk<T>(bt->ops[m], work_of<T>(bt->ops[m]), chunk, VAR_FAST, bt->streams[m]);
-      PB_HIP(bt->ctx, hipEventRecord(bt->joins[m], bt->streams[m]));
-      PB_HIP(bt->ctx, hipStreamWaitEvent(s, bt->joins[m], 0));
-    }
-    PB_HIP(bt->ctx, hipStreamEndCapture(s, &gr));
-    PB_HIP(bt->ctx, hipGraphInstantiate(&ex, gr, nullptr, nullptr, 0));
-    (void)hipGraphDestroy(gr);
-    it = bt->graphs.emplace(key, ex).first;
-  }
-  *out = it->second;
+  for (int m = 0; m < M; ++m) out[who[m]] = bt->hst[m];
   return PB_OK;
 }
 
@@ -2134,60 +2089,25 @@ int krylov_batch(pb_batch* bt, const std::vector<char>& active, const std::vecto
       return PB_OK;
     }
   }
-  // one launch over every member's tiles when they share the launch signature
-  if (flat_signature(bt) >= 0) return krylov_batch_flat<T>(bt, active, b, tol, maxiter, legacy, check_every, s, out);
-  const size_t M = bt->ops.size();
-  for (size_t m = 0; m < M; ++m) {
-    pb_op2d* op = bt->ops[m];
-    Work<T>& w = work_of<T>(op);
-    KState init{};
-    init.tol = tol[m];
-    init.maxiter = maxiter;
-    init.legacy = legacy;
-    init.phase = PH_INIT;
-    init.status = active[m] ? ST_RUN : ST_CONV;
-    bt->hst[m] = init;
-    if (active[m]) {
-      PB_HIP(bt->ctx, hipMemcpyAsync(w.S, bt->hst + m, sizeof(KState), hipMemcpyHostToDevice, s));
-      const dim3 grd = stencil_grid(op, op->ry);
-      const OpDev<T> d = opdev<T>(op);
-      InitIn<T> in{nullptr, false};
-      InitOut<T> o{b[m], w.r[0], w.rt, w.p[0], w.v[0], w.t, w.x, nullptr, false, 0.0, 0.0};
-      PB_DISPATCH(k_init5, T, op, grd, s, d, in, o, w.PB);
-      launch_a<T>(op, w, 1, s);
-    } else {   // parked: both state slots final, so every launch of the chunk is a no-op
-      PB_HIP(bt->ctx, hipMemcpyAsync(w.S, bt->hst + m, sizeof(KState), hipMemcpyHostToDevice, s));
-      PB_HIP(bt->ctx, hipMemcpyAsync(w.S + 1, bt->hst + m, sizeof(KState), hipMemcpyHostToDevice, s));
-    }
+  std::vector<int> kinds;
+  for (pb_op2d* op : bt->ops) kinds.push_back(kind_of(op));
+  if (kinds != bt->kinds) {   // the captured launches hold each kind's members and tiles
+    for (auto& kv : bt->graphs) (void)hipGraphExecDestroy(kv.second);
+    bt->graphs.clear();
+    bt->kinds = kinds;
   }
-  PB_LAUNCH_CHECK(bt->ctx);
-  const int chunk = std::max(2, (check_every > 0 ? check_every : 32) & ~1);
-  hipGraphExec_t ex = nullptr;
-  const bool graphs = graphs_enabled() && s != nullptr;
-  if (graphs) {
-    int rc = batch_graph<T>(bt, chunk, s, &ex);
+  KState parked{};
+  parked.status = ST_CONV;
+  out.assign(kinds.size(), parked);
+  std::map<int, std::vector<int>> by_kind;
+  for (size_t m = 0; m < kinds.size(); ++m) by_kind[kinds[m]].push_back((int)m);
+  for (const auto& kv : by_kind) {
+    bool any = false;
+    for (int m : kv.second) any = any || active[m];
+    if (!any) continue;
+    const int rc = krylov_batch_flat<T>(bt, kv.second, active, b, tol, maxiter, legacy, check_every, s, out);
     if (rc) return rc;
   }
-  long issued = 1;
-  for (;;) {
-    for (size_t m = 0; m < M; ++m)
-      PB_HIP(bt->ctx, hipMemcpyAsync(bt->hst + m, work_of<T>(bt->ops[m]).S + 1, sizeof(KState),
-                                     hipMemcpyDeviceToHost, s));
-    PB_HIP(bt->ctx, hipStreamSynchronize(s));
-    bool done = true;
-    for (size_t m = 0; m < M; ++m) done = done && st_final(bt->hst[m].status);
-    if (done) break;
-    if (issued > (long)maxiter + 2L * chunk + 2)
-      return pb_fail(bt->ctx, PB_ERR_STATE, "batch bicgstab: %ld iterations issued without final states", issued);
-    if (graphs) {
-      PB_HIP(bt->ctx, hipGraphLaunch(ex, s));
-    } else {
-      for (size_t m = 0; m < M; ++m) launch_chunk<T>(bt->ops[m], work_of<T>(bt->ops[m]), chunk, VAR_FAST, s);
-    }
-    PB_LAUNCH_CHECK(bt->ctx);
-    issued += chunk;
-  }
-  out.assign(bt->hst, bt->hst + M);
   return PB_OK;
 }
 
@@ -2250,15 +2170,8 @@ int batch_group_new(pb_ctx* ctx, pb_op2d* const* ops, int count, pb_batch** out)
     return pb_fail(ctx, PB_ERR_HIP, "pb_batch_create: %s failed", what);
   };
   for (int m = 0; m < count; ++m) {
-    hipStream_t st = nullptr;
-    hipEvent_t ev = nullptr;
-    if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) return fail("hipStreamCreate");
-    bt->streams.push_back(st);
-    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) return fail("hipEventCreate");
-    bt->joins.push_back(ev);
     if (alloc_work(ops[m])) return fail("workspace allocation");
   }
-  if (hipEventCreateWithFlags(&bt->fork, hipEventDisableTiming) != hipSuccess) return fail("hipEventCreate");
   void* hp = nullptr;
   if (hipHostMalloc(&hp, sizeof(KState) * count, hipHostMallocDefault) != hipSuccess) return fail("hipHostMalloc");
   bt->hst = (KState*)hp;
@@ -2273,15 +2186,10 @@ int batch_group_new(pb_ctx* ctx, pb_op2d* const* ops, int count, pb_batch** out)
 void batch_group_free(pb_batch* bt) {
   if (!bt) return;
   if (bt->ctx) (void)hipStreamSynchronize(bt->ctx->stream);
-  for (hipStream_t st : bt->streams) (void)hipStreamSynchronize(st);
   for (auto& kv : bt->graphs) (void)hipGraphExecDestroy(kv.second);
-  for (auto& kv : bt->flat_graphs) (void)hipGraphExecDestroy(kv.second);
   for (void* p : bt->mtab)
     if (p) (void)hipFree(p);
   if (bt->dstates) (void)hipFree(bt->dstates);
-  for (hipStream_t st : bt->streams) (void)hipStreamDestroy(st);
-  for (hipEvent_t ev : bt->joins) (void)hipEventDestroy(ev);
-  if (bt->fork) (void)hipEventDestroy(bt->fork);
   if (bt->hst) (void)hipHostFree(bt->hst);
   bt->records.release();
   delete bt;
@@ -2300,9 +2208,8 @@ extern "C" int pb_batch_destroy(pb_batch* bt) {
 //                      PB_SOLVE_F64_FAST solve of each member);
 //   PB_SOLVE_MIXED     FP32 Krylov (FP64 iterate) inside FP64 iterative
 //                      refinement to ||b - A x|| <= tol ||b||; the inner runs
-//                      of all members still refining share one graph per
-//                      chunk; a member whose refinement stalls finishes alone
-//                      in FP64.
+//                      of all members still refining share launches; a member
+//                      whose refinement stalls finishes alone in FP64.
 // Synchronous; infos[m] as pb_bicgstab_solve's.  Returns 0 when every member
 // converged, else the number of members that did not.
 extern "C" int pb_batch_solve(pb_batch* bt, const double* const* b, double* const* x, const pb_solve_opts* opts,
@@ -2331,8 +2238,7 @@ extern "C" int pb_batch_solve(pb_batch* bt, const double* const* b, double* cons
 }
 
 namespace {
-// one group: members solved together (flattened launches when they share the
-// launch signature, else one graph branch per member)
+// one group: members solved together
 int batch_group_solve(pb_batch* bt, const double* const* b, double* const* x, const pb_solve_opts* opts,
                       pb_solve_info* infos, hipStream_t s) {
   pb_ctx* ctx = bt->ctx;

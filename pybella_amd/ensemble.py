@@ -7,7 +7,7 @@ member).  Here every member keeps its own device state and operator, the
 members advance in lockstep (each with its own dt and time, exactly as its own
 ``do`` would), and at each of a step's two projections the solves of all
 members run as one batched solve (pb_batch_solve: resident launches for members
-that fit on the chip, else one hipGraph per chunk of iterations).  Every member's
+that fit on the chip, else shared launches per phase).  Every member's
 result equals its single-member GPU step with the same solver mode, bit for bit.
 """
 from __future__ import annotations

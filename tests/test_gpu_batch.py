@@ -163,6 +163,33 @@ def test_flattened_batch_equals_single_solves(ry, route):
         assert info["info"] == 0 and info["true_rel_resid"] <= 1e-8, info
 
 
+@pytest.mark.parametrize("mode", ["f64fast", "mixed"])
+def test_mixed_heights_by_launches(mode):
+    """Members of one size but several tile heights, by launches: kinds run in
+    turn, each with a graph of its own; after a uniform batch of the same
+    operators, and replayed over several solves."""
+    import torch
+    from pybella_amd import _abi
+    from pybella_amd.batch import BatchSolver
+    print(f"case batch mixed heights by launches {mode}", flush=True)
+    ops, bs = _systems([W.batch_member_bubble(129, 65, m) for m in range(12)])
+    ctx = ops[0].ctx
+    try:
+        for heights in ((4,), (2, 4, 8), (2, 3, 4, 5, 6, 8)):
+            for k, op in enumerate(ops):
+                op.set_tile(heights[k % len(heights)])
+            ctx.set_resident(_abi.PB_RESIDENT_OFF)
+            batch = BatchSolver(ops)
+            for _ in range(3):
+                xs, infos = batch.solve(bs, tol=1e-8, mode=mode)
+            ctx.set_resident(_abi.PB_RESIDENT_ON)
+            xr, ir = batch.solve(bs, tol=1e-8, mode=mode)
+            for x, i, y, j in zip(xs, infos, xr, ir):
+                assert i["info"] == 0 and i["iters"] == j["iters"] and torch.equal(x, y), (i, j)
+    finally:
+        ctx.set_resident(_abi.PB_RESIDENT_ON)
+
+
 def test_batch_of_more_tiles_than_are_resident_at_once():
     """Twelve members of 85 tiles and four smaller ones, one group: their 1046
     tiles go in two launches, each member's result bitwise that of its own
