@@ -262,8 +262,17 @@ def _nonhydrostasy(ud, step):
 
 
 def copy_fields(M: DeviceModel, src, dst):
-    """Contiguous device arrays copied in one launch on the model's stream."""
+    """Device arrays copied in one launch on the model's stream.  Any that is
+    not a contiguous FP64 array of its counterpart's shape goes through torch,
+    which converts or refuses."""
     src, dst = list(src), list(dst)
+    f64 = _torch().float64
+    for s, d in zip(src, dst):
+        if not (s.dtype is f64 and d.dtype is f64 and s.shape == d.shape and s.is_cuda and d.is_cuda
+                and s.is_contiguous() and d.is_contiguous()):
+            for a, b in zip(dst, src):
+                a.copy_(b)
+            return
     k = len(src)
     n = (C.c_int64 * k)(*[t.numel() for t in src])
     M.ctx.check(M.ctx.lib.pb_copy_fields(M.ctx.h, k, (C.c_void_p * k)(*[t.data_ptr() for t in src]),
