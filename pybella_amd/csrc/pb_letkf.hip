@@ -120,7 +120,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_letkf(LetkfArgs a, int chunk_w,
   using H = LetkfShape<KT>;
   constexpr int P = H::P, S = H::S;
   __shared__ double Ys[H::CAP * S];          // observation anomalies [position][member]
-  __shared__ double wv[H::CAP], dv[H::CAP];  // 1 / deviation (0: not observed, outside a wall); innovation
+  __shared__ double wv[H::CAP], dv[H::CAP];  // 1 / deviation (root of the variance's size; 0: not observed, outside a wall); innovation
   const int lane = threadIdx.x, wave = threadIdx.y, tid = lane + 64 * wave;
   const int m = lane % 16, grp = lane / 16;
   const int tiles_x = (a.nx + P - 1) / P;
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_letkf(LetkfArgs a, int chunk_w,
   // Y^T W Y and Y^T W d over the windows, by attribute, by chunks of
   // chunk_w window columns and of chunk_h rows of the block's window union
   for (int at = 0; at < a.attrs; ++at) {
-    const double idev = 1.0 / sqrt(covar ? covar[at] : 1.0);
+    const double var = covar ? covar[at] : 1.0, idev = 1.0 / sqrt(fabs(var));
     for (int c0 = 0; c0 < a.ox; c0 += chunk_w) {
       const int cw = min(chunk_w, a.ox - c0), RW = P + cw - 1;
       for (int r0 = 0; r0 < kWaves + a.oy - 1; r0 += chunk_h) {
@@ -185,9 +185,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_letkf(LetkfArgs a, int chunk_w,
           const bool ok = s < n;
           const int pos = ok ? (wave + w0 + q - r0) * RW + c : 0;
           // both operands carry the root of the weight, so Pa is exactly
-          // symmetric; a negative weight's sign goes with one of them
+          // symmetric; the sign of a negative weight / variance goes with one of them
           const double rl = sqrt(fabs(L));
-          const bool neg = L < 0.0;
+          const bool neg = (L < 0.0) != (var < 0.0);
           c += 4;
           while (c >= cw) {
             c -= cw;

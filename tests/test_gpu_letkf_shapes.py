@@ -2,8 +2,8 @@
 LETKF oracle (oracle/letkf.py analyse_grid): 2, 16, 17 and 32 members (one
 and two 16-member tiles, full and nearly empty), grids that leave rows and
 columns of the last block unused, windows larger than the staging area in
-rows and in columns, one attribute and more than sixteen, walls on both axes,
-accurate observations (a condition number of ~1e6), none at all, and NaN where
+rows and in columns, one attribute and more than sixteen, walls on both axes, on either
+and on none, a negative variance (taken as any other number), accurate observations (a condition number of ~1e6), none at all, and NaN where
 nothing is observed.
 
 Tolerance: the analysis is x_mean + Wa X with |Wa| ~ 1; Wa's relative error is
@@ -25,7 +25,8 @@ pytestmark = pytest.mark.gpu
     (17, 2, 13, 6, 5, 5, (1, 1), 0.01, 1e-10), (32, 3, 19, 15, 13, 9, (0, 1), 0.01, 1e-10),
     (7, 2, 30, 33, 21, 31, (1, 1), 0.01, 1e-10), (3, 1, 300, 5, 291, 3, (0, 0), 0.01, 1e-10),
     (20, 1, 200, 4, 195, 1, (0, 1), 0.01, 1e-10), (5, 19, 12, 10, 3, 3, (0, 1), 0.01, 1e-10),
-    (16, 2, 20, 11, 7, 7, (0, 1), 1e-6, 4e-9), (12, 1, 16, 16, 1, 1, (0, 0), 0.01, 1e-10)])
+    (16, 2, 20, 11, 7, 7, (0, 1), 1e-6, 4e-9), (12, 1, 16, 16, 1, 1, (0, 0), 0.01, 1e-10),
+    (16, 3, 18, 13, 5, 7, (1, 0), 0.01, 1e-10), (9, 2, 14, 11, 3, 3, (0, 0), -40.0, 1e-10)])
 def test_letkf_shapes(k, attrs, nx, ny, ox, oy, walls, var, tol):
     import torch
     from pybella_amd import _abi
@@ -37,6 +38,12 @@ def test_letkf_shapes(k, attrs, nx, ny, ox, oy, walls, var, tol):
     covar = var * rng.uniform(0.5, 2.0, attrs)
     loc = rng.random((ox, oy))
     bc = ol.boundary_mask((nx, ny), (not walls[0], not walls[1]), (ox - 1) // 2, (oy - 1) // 2)
+    if walls == (1, 0):
+        # beyond an x wall nothing is observed; the reference pads x with 0 and
+        # then the periodic y with 1, which gives the corners back their weight
+        px, py = (ox - 1) // 2, (oy - 1) // 2
+        assert (bc[:px, :py] == 1).all() and (bc[:px, py:-py] == 0).all()
+        bc[:px], bc[-px:] = 0.0, 0.0
     ref = ol.analyse_grid(state, obs, mask, covar, loc, bc, ox, oy, 1.05)
     ctx = _abi.default_context()
     dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
