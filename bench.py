@@ -15,7 +15,7 @@ resident in HBM before the timed region; every timed step does all of that
 work.
 
 Printed: ONE JSON line with the contract fields plus ``roofline`` (dominant
-kernel, HBM-bound) and ``cpu_baseline`` (the C restatement of the reference's
+kernel of the launch-per-phase path, HBM-bound) and ``cpu_baseline`` (the C restatement of the reference's
 serial matvec + BiCGStab, oracle/c/pb_oracle.c, on a bounded sample).
 """
 from __future__ import annotations
@@ -45,8 +45,10 @@ KERNEL_NAMES = {0: "matvec", 1: "bicg_fast_A_pupdate_matvec", 2: "bicg_B_s_matve
 
 SOLVER_NAMES = {
     "mixed": "plain BiCGStab, FP32 Krylov (FP64 iterate) in FP64 iterative refinement",
-    "f64": "plain BiCGStab FP64 (reference semantics, 3 launches/iteration)",
-    "f64fast": "plain BiCGStab FP64 (rho, ||r|| from s/t dots, 2 launches/iteration)",
+    "f64": "plain BiCGStab FP64 (reference semantics, three phases per iteration; the run in one launch "
+           "where its tiles fit on the chip, else a launch per phase)",
+    "f64fast": "plain BiCGStab FP64 (rho, ||r|| from s/t dots, two phases per iteration; the run in one "
+               "launch where its tiles fit on the chip, else a launch per phase)",
     "f64fused": "plain BiCGStab FP64 (as f64fast; r~.v as u.p with u = A^T r~, 1 launch/iteration)",
     "nn": "learned preconditioner: FP64 flexible GMRES preconditioned by the FP32 two-branch multigrid cycle "
           "whose coarse level (65x33 nodes) the BF16 network solves; plain BiCGStab FP64 only past the budget",
@@ -190,8 +192,8 @@ def _node_null_rel(p, q):
 
 def bench_ensemble(args, count=16, nx=161, ny=81, nsteps=6):
     """Member time steps per second of a rising-bubble ensemble on one grid:
-    the members stepped in lockstep with their solves batched (one graph per
-    chunk of iterations over all members), beside the same members stepped
+    the members stepped in lockstep with their solves batched (all members'
+    runs on the chip in shared launches), beside the same members stepped
     one after the other as the reference's member loop does
     (src/__main__.py:223-254), both with the FP64 fast solver."""
     import copy
@@ -596,7 +598,8 @@ def bench_batch(args, sizes=((129, 65), (257, 129), (513, 257), (1025, 513))):
     """64 rising-bubble pressure solves (members_per_size at each grid size,
     seeded bubble amplitude, centre and radius), each member's operator and
     right-hand side from its own projection step; all solved by one batched
-    solve (one hipGraph per chunk of iterations over every member) vs the
+    solve (runs on the chip in shared launches where they fit, else a
+    hipGraph per chunk of iterations over every member of a group) vs the
     same solves one after the other.  Tile heights come from the autotuner,
     one per grid size."""
     import torch
@@ -625,8 +628,8 @@ def bench_batch(args, sizes=((129, 65), (257, 129), (513, 257), (1025, 513))):
             if (mx, my) == (nx, ny):
                 op.set_tile(best)
     batch = BatchSolver(ops)
-    # one tile height for the whole batch lets it run one launch over every
-    # member's tiles per phase; the autotuner times the batch itself
+    # one tile height for the whole batch lets its members share launches; the
+    # autotuner times the batch itself
     per_size = {v["rows_per_thread"] for v in tiles.values()}
     btable = {}
     from pybella_amd.autotune import CANDIDATES
@@ -733,7 +736,7 @@ def main():
     ap.add_argument("--tile", type=int, default=4, help="rows per thread for --kernel-only")
     ap.add_argument("--workload", default="2d", choices=["2d", "3d", "batch", "step", "timestep", "ensemble"],
                     help="3d: the isolated 257x129x129 27-point solve; batch: 64 uneven rising-bubble "
-                         "solves in one graph per chunk; step: whole projection steps (the drop-in "
+                         "solves in shared launches; step: whole projection steps (the drop-in "
                          "impl_part) at 1025x513; timestep: rising-bubble time steps/s at 161x81 and "
                          "1025x513; ensemble: 16 rising-bubble members stepped with batched solves (each its "
                          "own JSON line, not the metric)")
@@ -900,8 +903,9 @@ def main():
     x_plain = x.clone()
     op.set_tile(tiles[plain]["rows_per_thread"])
 
-    # roofline of the plain BiCGStab's dominant launch: HIP events around every
-    # launch inside a real solve, and on pattern-filled vectors beside it
+    # roofline of the dominant launch of plain BiCGStab by launches, the path of
+    # grids too large for the chip (the plain solves timed above run resident): HIP
+    # events inside a real solve, and on pattern-filled vectors beside it
     n = grid.nx * grid.ny
     kt = {k: op.time_kernel(k, "f64", args.kernel_reps) for k in (0, 1, 2, 3)}
     op.assemble(phys, dt, rho, rhoY, rho, rhoY, dS)
@@ -914,7 +918,8 @@ def main():
     alg = KERNEL_WORDS[dom] * 8 * n + KERNEL_XBYTES.get(dom, 0) * n
     achieved = alg / (in_solve[dom][0] * 1e-6) / 1e9
     achieved_syn = alg / (kt[dom] * 1e-6) / 1e9
-    roof = {"bound": "hbm", "kernel": KERNEL_NAMES[dom], "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
+    roof = {"bound": "hbm", "kernel": KERNEL_NAMES[dom],
+            "path": "plain BiCGStab by launches (grids too large to stay on the chip)", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
             "avg_us": round(in_solve[dom][0], 3), "timed_in_solve_launches": in_solve[dom][1], "alg_bytes": alg,
             "synthetic_state": {"avg_us": round(kt[dom], 3), "achieved": round(achieved_syn, 1),

@@ -173,10 +173,13 @@ __global__ void k_clear_words(long n, u64* w) {
   for (long g = blockIdx.x * (long)blockDim.x + threadIdx.x; g < n; g += (long)gridDim.x * blockDim.x) w[g] = 0;
 }
 
-// One tile of one member for a whole run.  Blocks take their tile from the
-// ticket counter in the order they start, so a batch larger than the chip is
-// worked off in member order: the blocks of the first unfinished member are
-// always among those that have started or start next.
+// One tile of one member for a whole run.  All blocks of a launch are resident
+// at once (run_jobs), so any tile order is right; each takes its tile from the
+// ticket counter in the order the blocks start.  Tiles by block index instead,
+// us per iteration, exact / fast: 161x81 (18 tiles) 8.9 / 6.7 -> 9.5 / 7.2,
+// 257x129 (45) 9.9 / 7.4 -> 10.5 / 7.7; above 96 tiles, where a few blocks form
+// the class sums for all, the index is the better order (513x257, 153 tiles:
+// 13.9 / 10.0 -> 11.8 / 9.0).
 template <typename T, bool CROSS, bool CENTER, int RY, bool EXACT, int MINB>
 __global__ __launch_bounds__(NTHR, MINB) void k_resident(const RMember<T>* __restrict__ tab, int nmem, u32* ticket,
                                                    u32 ticket0) {
