@@ -732,9 +732,11 @@ ResKernel<T> pick_kind(bool cross, bool center) {
   return center ? k_resident<T, false, true, RY, EXACT, MINB> : k_resident<T, false, false, RY, EXACT, MINB>;
 }
 // The kernel of a tile height for grids of ``nb`` tiles.  Blocks per CU that
-// the registers are to leave room for: two; three up to 3-row tiles, which
-// need few, and for 4-row tiles on grids with more than two tiles per CU
-// (1025x513: 561), where some of the FP64 kinds then spill.
+// the registers are to leave room for: two; three up to 3-row tiles, and for
+// 4-row tiles on grids with more than two tiles per CU (1025x513: 561).  Spilled
+// VGPRs of the FP64 kinds: 2 rows 0-3, 3 rows 2-34, 4 rows 26-79 with three
+// blocks and none with two, 5 rows 0-25, 6 rows 3-59, 8 rows (one block) none;
+// no FP32 kind spills.
 template <typename T, bool EXACT>
 ResKernel<T> pick(int ry, bool cross, bool center, bool many) {
   switch (ry) {
