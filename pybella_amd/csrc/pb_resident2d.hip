@@ -11,8 +11,8 @@
 // MB at 1025x513), and what blocks exchange is one ring of edge values and a
 // few sums per stencil.  FP64 at 4-row tiles, us per iteration, launches ->
 // resident: two phases 14.0 -> 6.7 (161x81), 13.6 -> 9.8 (513x257), 24.7 ->
-// 15.0 (1025x513); the exact variant's three 18.7 -> 9.1, 18.5 -> 13.5, 28.5 ->
-// 19.6.  What is left is latency: per phase at 161x81 about 1.5 us for the
+// 15.3 (1025x513); the exact variant's three 18.7 -> 9.1, 18.5 -> 13.5, 28.5 ->
+// 19.3.  What is left is latency: per phase at 161x81 about 1.5 us for the
 // hand-over and 1.9 us for the chain combine, stencil, sums, scalars of one
 // tile.  (x updated in the chain instead of behind the hand-over: 7.3; eight
 // waves per tile instead of four: 6.8; waves that sleep between polls: 7.3.)
